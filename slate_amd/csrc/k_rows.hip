@@ -1,6 +1,8 @@
 // k_rows.hip -- row-wise kernels: RMSNorm (+residual), SiLU*mul, RoPE with
 // KV append, embedding gather, greedy argmax, ragged-batch packing and the
 // small f32 matmuls behind the vtable's matvec / linear_batch.
+#include <type_traits>
+
 #include "launch.h"
 #include "act16.h"
 #include "rowops.h"
@@ -725,43 +727,161 @@ int launch_mm_f32(float* Y, const float* X, const float* W, int B, int M, int K,
     return 0;
 }
 
-// C[b, n] = sum_k X[b, k] * W[k, n] (W is [K, N] for linear_batch, backend.h:58-61).
-// A workgroup owns 64 columns and LB_ROWS batch rows: lanes over n
-// (coalesced W rows), the four waves over k (k = wave mod 4), each W element
-// loaded once for all the rows, the waves' sums combined in LDS in a fixed
-// order.
-constexpr int LB_ROWS = 8;
-__global__ __launch_bounds__(256) void linear_batch_kernel(float* __restrict__ C, const float* __restrict__ X,
-                                                           const float* __restrict__ W, int B, int K, int N) {
-    __shared__ float red[4][LB_ROWS][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int n = blockIdx.x * 64 + lane;
-    const int b0 = blockIdx.y * LB_ROWS;
-    const int nb = min(LB_ROWS, B - b0);
-    float acc[LB_ROWS];
+// C[b, n] = sum_k X[b, k] * W[k, n] (W is [K, N] for linear_batch,
+// backend.h:58-61) on the f32 MFMA (16 batch rows x 16 columns x 4 k, exact
+// f32 products and sums).
+//
+// A workgroup owns 16 * NC columns and 16 * BT batch rows.  Its NW waves take
+// the 16-element units of K in turn (unit u to wave u mod NW, four units'
+// loads issued before any is used); of a unit, lane (j, g) = (lane & 15,
+// lane >> 4) loads X[row j][4g .. 4g+3] and, for step s < 4, columns
+// NC*j .. NC*j+NC-1 of row 4g + s of W, so every load of W is four runs of
+// 64 * NC bytes and a step's NC MFMAs (column NC*j + e for e < NC) need no
+// shuffle.  The waves' sums meet in LDS and are added in wave order.
+//
+// What bounds it: reading W once from 8192 columns on (4096 x 16384 at B 16:
+// 53 us, 5.1 TB/s), below that latency and the MFMAs of the few CUs that have
+// a workgroup.  The form before (a column per lane, four waves over k, one
+// dependent load of W and one of X per batch row and k) took 208 us per call
+// for B 16, K 1024, N 4096, this one 6.8 us.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // rows start on any float
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float fx4 __attribute__((ext_vector_type(4)));
+
+template <int NC, int BT, int NW, int AHEAD>
+__global__ __launch_bounds__(64 * NW) void linear_batch_kernel(float* __restrict__ C, const float* __restrict__ X,
+                                                               const float* __restrict__ W, int B, int K, int N) {
+    static_assert(NC == 1 || NC == 2 || NC == 4, "one, two or four columns per lane");
+    constexpr int COLS = 16 * NC, ROWS = 16 * BT;
+    __shared__ float red[NW][ROWS][COLS];
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int cg = blockIdx.x;
+    if (NC == 1) {
+        // 64-byte runs of W: the two groups of a 128-byte line on one XCD
+        // (workgroups go to the eight XCDs in turn)
+        const int q = gridDim.x & ~15;
+        if (cg < q) cg = (((cg >> 4) << 3 | (cg & 7)) << 1) | ((cg >> 3) & 1);
+    }
+    const int c0 = cg * COLS, b0 = blockIdx.y * ROWS;
+    // the lane's first column: the last lanes of the last group step back to
+    // whole loads, so a column may have two lanes with the same sums (N >= NC)
+    const int cl = min(c0 + NC * j, N - NC);
+    const int units = (K + 15) / 16, full = K / 16;
+    fx4 acc[BT][NC];
 #pragma unroll
-    for (int i = 0; i < LB_ROWS; ++i) acc[i] = 0.f;
-    if (n < N) {
-        for (int k = wv; k < K; k += 4) {
-            const float w = W[(size_t)k * N + n];
+    for (int n = 0; n < BT; ++n)
 #pragma unroll
-            for (int i = 0; i < LB_ROWS; ++i)
-                if (i < nb) acc[i] = __builtin_fmaf(X[(size_t)(b0 + i) * K + k], w, acc[i]);
+        for (int e = 0; e < NC; ++e) acc[n][e] = fx4{0.f, 0.f, 0.f, 0.f};
+    // rows past B repeat the last one: their sums are never stored
+    const float* xr[BT];
+#pragma unroll
+    for (int n = 0; n < BT; ++n) xr[n] = X + (size_t)min(b0 + 16 * n + j, B - 1) * K + 4 * g;
+    const float* wr = W + (size_t)(4 * g) * N + cl;
+
+    struct Unit { fx4 x[BT]; float w[4][NC]; };
+    auto load = [&](Unit& t, int u) {              // a whole unit, u < full
+        const float* wu = wr + (size_t)u * 16 * N;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if constexpr (NC == 4) {
+                const f4u v = *(const f4u*)(wu + (size_t)s * N);
+                t.w[s][0] = v.x; t.w[s][1] = v.y; t.w[s][2] = v.z; t.w[s][3] = v.w;
+            } else if constexpr (NC == 2) {
+                const f2u v = *(const f2u*)(wu + (size_t)s * N);
+                t.w[s][0] = v.x; t.w[s][1] = v.y;
+            } else {
+                t.w[s][0] = wu[(size_t)s * N];
+            }
         }
-    }
 #pragma unroll
-    for (int i = 0; i < LB_ROWS; ++i) red[wv][i][lane] = acc[i];
-    __syncthreads();
-    if (wv == 0 && n < N) {
-        for (int i = 0; i < nb; ++i)
-            C[(size_t)(b0 + i) * N + n] = (red[0][i][lane] + red[1][i][lane]) + (red[2][i][lane] + red[3][i][lane]);
+        for (int n = 0; n < BT; ++n) {
+            const f4u v = *(const f4u*)(xr[n] + 16 * u);
+            t.x[n] = fx4{v.x, v.y, v.z, v.w};
+        }
+    };
+    auto mul = [&](const Unit& t) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int n = 0; n < BT; ++n)
+#pragma unroll
+                for (int e = 0; e < NC; ++e)
+                    acc[n][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.x[n][s], t.w[s][e], acc[n][e], 0, 0, 0);
+    };
+    // n units' loads in flight, then their products: AHEAD at a time, the
+    // rest by powers of two (no load is repeated or wasted)
+    int u = wv;
+    auto batch = [&](auto n) {
+        constexpr int NU = decltype(n)::value;
+        Unit t[NU];
+#pragma unroll
+        for (int i = 0; i < NU; ++i) load(t[i], u + i * NW);
+#pragma unroll
+        for (int i = 0; i < NU; ++i) mul(t[i]);
+        u += NU * NW;
+    };
+    while (u + (AHEAD - 1) * NW < full) batch(std::integral_constant<int, AHEAD>{});
+    if constexpr (AHEAD > 4)
+        if (u + 3 * NW < full) batch(std::integral_constant<int, 4>{});
+    if constexpr (AHEAD > 2)
+        if (u + NW < full) batch(std::integral_constant<int, 2>{});
+    if (u < full) batch(std::integral_constant<int, 1>{});
+    if (units > full && wv == full % NW) {         // the last K % 16 elements, zeros past them
+        Unit t;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int k = 16 * full + 4 * g + s;
+#pragma unroll
+            for (int e = 0; e < NC; ++e) t.w[s][e] = k < K ? W[(size_t)k * N + cl + e] : 0.f;
+#pragma unroll
+            for (int n = 0; n < BT; ++n) t.x[n][s] = k < K ? xr[n][16 * full + s] : 0.f;
+        }
+        mul(t);
     }
+    // D[i][j]: lane (j, g) holds rows 4g .. 4g+3 of its column
+#pragma unroll
+    for (int n = 0; n < BT; ++n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < NC; ++e)
+                if (cl + e >= c0) red[wv][16 * n + 4 * g + i][cl + e - c0] = acc[n][e][i];
+    __syncthreads();
+    const int nw = min(NW, units);                 // waves that had units
+    for (int o = threadIdx.x; o < ROWS * COLS; o += 64 * NW) {
+        const int r = o / COLS, c = o % COLS;
+        if (b0 + r >= B || c0 + c >= N) continue;
+        float v = red[0][r][c];
+        for (int w = 1; w < nw; ++w) v += red[w][r][c];
+        C[(size_t)(b0 + r) * N + c0 + c] = v;
+    }
+}
+
+template <int NC, int BT, int NW, int AHEAD>
+static void launch_linear(float* C, const float* X, const float* W, int B, int K, int N, hipStream_t s) {
+    const dim3 grid((N + 16 * NC - 1) / (16 * NC), (B + 16 * BT - 1) / (16 * BT));
+    hipLaunchKernelGGL((linear_batch_kernel<NC, BT, NW, AHEAD>), grid, dim3(64 * NW), 0, s, C, X, W, B, K, N);
+}
+
+// Columns per lane: one while that gives at most one workgroup per CU, then
+// two, then four (wider runs of W, fewer reads of X): K 1024, N 4096, B 16
+// takes 6.8 us with one, 8.8 with two, 11.2 with four; K 2048, N 8192 16.7 /
+// 15.3 / 19.7; K 4096, N 16384 94 / 62 / 53 us.  Waves and units in flight
+// keep two workgroups' registers on a CU.
+template <int BT, int NW>
+static void launch_linear_cols(float* C, const float* X, const float* W, int B, int K, int N, hipStream_t s) {
+    constexpr int A = BT == 1 ? 4 : 2;
+    if (N <= 16 * 256) launch_linear<1, BT, NW, A>(C, X, W, B, K, N, s);
+    else if (N <= 32 * 256) launch_linear<2, BT, NW, A>(C, X, W, B, K, N, s);
+    else launch_linear<4, BT, BT == 1 ? 16 : 8, BT == 4 ? 1 : 2>(C, X, W, B, K, N, s);
 }
 
 int launch_linear_batch(float* C, const float* X, const float* W, int B, int K, int N, hipStream_t s) {
     if (B <= 0 || N <= 0) return 0;
-    hipLaunchKernelGGL(linear_batch_kernel, dim3((N + 63) / 64, (B + LB_ROWS - 1) / LB_ROWS), dim3(256), 0, s, C,
-                       X, W, B, K, N);
+    if (B <= 16) launch_linear_cols<1, 16>(C, X, W, B, K, N, s);
+    else if (B <= 32) launch_linear_cols<2, 16>(C, X, W, B, K, N, s);
+    else launch_linear_cols<4, 8>(C, X, W, B, K, N, s);
     SH_CHECK_LAUNCH();
     return 0;
 }
