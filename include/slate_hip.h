@@ -156,9 +156,10 @@ int   slate_hip_dequant_q8_0(float* dst, const void* A_q8, int64_t n);          
 /* Tiled Q8_0: the same bytes regrouped into 16-row x 256-element tiles of
  * 4352 bytes (the eight d of each row, then the int8 weights in the order
  * the matmul lanes read them); rows past M and blocks past K/32 are zero.
- * matmul_q8_0 regroups into backend scratch on every call; callers that
- * keep weights resident tile them once with q8_0_tile (device src, row
- * layout, into dst of q8_0_tiled_bytes) and call matmul_q8_0_tiled. */
+ * From two rows on, matmul_q8_0 regroups into backend scratch on every call;
+ * callers that keep weights resident tile them once with q8_0_tile (device
+ * src, row layout, into dst of q8_0_tiled_bytes) and call matmul_q8_0_tiled
+ * (same results). */
 int64_t slate_hip_q8_0_tiled_bytes(int M, int K);
 int   slate_hip_q8_0_tile(void* dst_tiled, const void* src_q8, int M, int K);
 int   slate_hip_matmul_q8_0_tiled(float* Y, const void* A_tiled, const float* X, int B, int M, int K);

@@ -218,6 +218,8 @@ inline size_t act8_bytes(int rows_pad, int K) {
 }
 int launch_act8_from_f32(const Act8& a, const float* X, int64_t ldx, hipStream_t s);
 int make_act8(Act8& a, int B, int K, int slot);
+// One row of x (16-byte aligned) against M rows of either layout.
+int launch_q8_gemv(const void* W, bool tiled, int M, int K, const float* x, float* y, hipStream_t s);
 // Up to three TILED Q8_0 tensors sharing one input (targets and partial
 // layout as launch_q4k).  fixed_splits > 0 forces that split count (a group
 // that also holds Q4_K tensors must write the same partials); otherwise the

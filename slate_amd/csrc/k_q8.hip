@@ -51,47 +51,80 @@ int launch_dequant_q8(float* dst, const void* src, int64_t n_blocks, hipStream_t
 // so MFMA K step t (block t of the group) takes from lane group g the 8
 // weights 8g..8g+7 of the block, and each load of a wave is one contiguous
 // 256- or 1024-byte run.  The bytes are the row layout's, regrouped.
+//
+// A workgroup regroups TG groups of one tile through LDS: the rows' bytes come
+// in as unaligned 16-byte loads (1088 contiguous bytes per row), the units go
+// out as contiguous 16-byte stores, so each side moves whole lines once.
+// matmul_q8_0 at 16 rows: 4096 x 4096 25.8 us per call, 14336 x 4096 50.5 us;
+// 47.2 and 129 us when each thread gathered its unit byte by byte from global
+// memory.  (The matmul on the row layout itself, by unaligned 8-byte loads
+// per lane: 23.4 and 54.9 us, but 43 against 23.5 us for 1024 x 2048 at 65
+// rows and 468 against 223 us for 14336 x 4096 at 512 rows.)
+struct __attribute__((packed, aligned(1))) U16B { uint32_t x, y, z, w; };
+struct __attribute__((packed, aligned(1))) H16 { uint16_t v; };
+constexpr int Q8T_GROUPS = 4;
 __global__ __launch_bounds__(256) void q8_tile_kernel(uint4* __restrict__ dst, const uint8_t* __restrict__ src,
-                                                      int M, int K, int ngrp, int64_t units) {
-    const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (u >= units) return;
-    const int64_t tb = u / (Q8_TB / 16);
-    const int w = (int)(u - tb * (Q8_TB / 16));
-    const int64_t tile = tb / ngrp;
-    const int kb = (int)(tb - tile * ngrp);
-    const int nb32 = K / Q8_ELEMS;
-    union { uint4 v; uint8_t b[16]; } o;
-    if (w < 16) {
-        const int64_t row = tile * 16 + w;
-        for (int t = 0; t < 8; ++t) {
-            const int blk = kb * 8 + t;
-            const bool in = row < M && blk < nb32;
-            const uint8_t* p = src + (row * nb32 + blk) * Q8_BYTES;
-            o.b[2 * t] = in ? p[0] : 0;
-            o.b[2 * t + 1] = in ? p[1] : 0;
+                                                      int M, int nb32, int ngrp) {
+    constexpr int SEG = Q8T_GROUPS * 8 * Q8_BYTES, UNITS = SEG / 16;   // a row's bytes and 16-byte pieces
+    constexpr int PITCH = SEG + 16;
+    __shared__ __align__(16) uint8_t s[16 * PITCH];
+    const int kb0 = blockIdx.x * Q8T_GROUPS, tile = blockIdx.y;
+    const int ng = min(Q8T_GROUPS, ngrp - kb0);
+    const size_t rb = (size_t)nb32 * Q8_BYTES;
+    const int left = (int)min((size_t)SEG, rb - (size_t)kb0 * 8 * Q8_BYTES);   // bytes of a row from group kb0
+    for (int i = threadIdx.x; i < 16 * UNITS; i += 256) {
+        const int r = i / UNITS, o = 16 * (i - r * UNITS);
+        const int64_t row = (int64_t)tile * 16 + r;
+        union { uint4 v; uint16_t h[8]; } t;
+        t.v = make_uint4(0u, 0u, 0u, 0u);
+        if (row < M) {
+            const uint8_t* p = src + row * rb + (size_t)kb0 * 8 * Q8_BYTES + o;
+            if (o + 16 <= left) {
+                const U16B u = *(const U16B*)p;
+                t.v = make_uint4(u.x, u.y, u.z, u.w);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    if (o + 2 * k < left) t.h[k] = ((const H16*)(p + 2 * k))->v;
+            }
         }
-    } else {
-        const int c = (w - 16) >> 6, l = (w - 16) & 63;
-        const int j = l & 15, g = l >> 4;
-        const int64_t row = tile * 16 + j;
-        for (int h = 0; h < 2; ++h) {
-            const int blk = kb * 8 + 2 * c + h;
-            const bool in = row < M && blk < nb32;
-            const uint8_t* p = src + (row * nb32 + blk) * Q8_BYTES + 2 + 8 * g;
-            for (int e = 0; e < 8; ++e) o.b[8 * h + e] = in ? p[e] : 0;
-        }
+        *(uint4*)(s + r * PITCH + o) = t.v;
     }
-    dst[u] = o.v;
+    __syncthreads();
+    constexpr int TU = Q8_TB / 16;                 // units of a group
+    uint4* out = dst + ((size_t)tile * ngrp + kb0) * TU;
+    for (int i = threadIdx.x; i < ng * TU; i += 256) {
+        const int kg = i / TU, w = i - kg * TU;
+        union { uint4 v; uint16_t h[8]; } t;
+        if (w < 16) {                              // row w's eight d
+            const uint8_t* p = s + w * PITCH + kg * 8 * Q8_BYTES;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) t.h[k] = *(const uint16_t*)(p + k * Q8_BYTES);
+        } else {
+            const int c = (w - 16) >> 6, l = (w - 16) & 63, j = l & 15, g = l >> 4;
+            const uint8_t* p = s + j * PITCH + (kg * 8 + 2 * c) * Q8_BYTES + 2 + 8 * g;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                t.h[k] = *(const uint16_t*)(p + 2 * k);
+                t.h[4 + k] = *(const uint16_t*)(p + Q8_BYTES + 2 * k);
+            }
+        }
+        out[i] = t.v;
+    }
 }
 
 size_t q8_tiled_bytes(int M, int K) { return (size_t)((M + 15) / 16) * q8_groups(K) * Q8_TB; }
 
 int launch_q8_tile(void* dst, const void* src, int M, int K, hipStream_t s) {
-    const int ngrp = q8_groups(K);
-    const int64_t units = (int64_t)((M + 15) / 16) * ngrp * (Q8_TB / 16);
-    if (units == 0) return 0;
-    hipLaunchKernelGGL(q8_tile_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, (uint4*)dst,
-                       (const uint8_t*)src, M, K, ngrp, units);
+    const int ngrp = q8_groups(K), tiles = (M + 15) / 16;
+    if (M <= 0 || ngrp == 0) return 0;
+    for (int t0 = 0; t0 < tiles; t0 += 65535) {    // grid rows
+        const int nt = std::min(65535, tiles - t0);
+        hipLaunchKernelGGL(q8_tile_kernel, dim3((ngrp + Q8T_GROUPS - 1) / Q8T_GROUPS, nt), dim3(256), 0, s,
+                           (uint4*)dst + (size_t)t0 * ngrp * (Q8_TB / 16),
+                           (const uint8_t*)src + (size_t)t0 * 16 * (K / Q8_ELEMS) * Q8_BYTES, M - t0 * 16,
+                           K / Q8_ELEMS, ngrp);
+    }
     SH_CHECK_LAUNCH();
     return 0;
 }
@@ -358,6 +391,106 @@ __global__ __launch_bounds__(64 * WAVES) void q8_mm_kernel(Q4kTargets tg, const 
                     for (int i = 0; i < 4; ++i) o[(int64_t)((at0 + n) * 16 + 4 * g + i) * ldo + row] = acc[r][n][i];
         }
     }
+}
+
+// One activation row (quant.c:126-133, q8_0_matvec) on the vector ALUs: a
+// workgroup owns R weight rows and all of K; thread t owns half a block (16
+// weights of every row), its 16 values of x in registers for all R rows, and
+// issues the R rows' loads before any arithmetic.  In the row layout that is
+// one unaligned 16-byte load and the block's d per row (a wave reads 1088
+// contiguous bytes), in the TILED layout two 8-byte loads and d (the R rows'
+// loads together read whole lines).  Sums: twice 8 products in f32, times d, then
+// DPP over the wave and LDS over the waves in wave order: deterministic, and
+// the same bits from both layouts.
+//
+// Bound by HBM and by the latency of the one round of loads.  Per call at
+// 4096 x 4096, row layout: 46.9 us as regrouping pass + operand + matmul +
+// split sum, 5.7 us as one kernel; TILED 11.6 us as operand + matmul + split
+// sum, 6.9 us; 14336 x 4096: 129 and 17.7 us, 12.3 (5.1 TB/s) and 16.5 us.
+constexpr int Q8V_WAVES = 8;
+template <int R, bool TILED>
+__global__ __launch_bounds__(64 * Q8V_WAVES) void q8_gemv_kernel(const uint8_t* __restrict__ W,
+                                                                  const float* __restrict__ x,
+                                                                  float* __restrict__ y, int M, int nhalf) {
+    __shared__ float red[Q8V_WAVES][R];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, m0 = blockIdx.x * R;
+    const int nb32 = nhalf >> 1, ngrp = (nb32 + 7) >> 3;
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+    for (int hb = threadIdx.x; hb < nhalf; hb += blockDim.x) {
+        const int blk = hb >> 1, h = hb & 1;
+        uint4 q[R];
+        uint32_t d[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int m = min(m0 + r, M - 1);
+            if (TILED) {
+                // lane groups 2h and 2h + 1 of row m's block (layout above)
+                const uint8_t* tb = W + ((size_t)(m >> 4) * ngrp + (blk >> 3)) * Q8_TB;
+                const int t = blk & 7, j = m & 15;
+                const uint8_t* p = tb + 256 + 1024 * (t >> 1) + 16 * (32 * h + j) + 8 * (t & 1);
+                const uint2 a = *(const uint2*)p, b = *(const uint2*)(p + 256);
+                q[r] = make_uint4(a.x, a.y, b.x, b.y);
+                d[r] = *(const uint16_t*)(tb + 16 * j + 2 * t);
+            } else {
+                const uint8_t* p = W + ((size_t)m * nb32 + blk) * Q8_BYTES;
+                const U16B v = *(const U16B*)(p + 2 + 16 * h);
+                q[r] = make_uint4(v.x, v.y, v.z, v.w);
+                d[r] = ((const H16*)p)->v;
+            }
+        }
+        float xv[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 v = *(const float4*)(x + (size_t)hb * 16 + 4 * i);
+            xv[4 * i] = v.x; xv[4 * i + 1] = v.y; xv[4 * i + 2] = v.z; xv[4 * i + 3] = v.w;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t w[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
+            float s[2] = {0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    s[i >> 1] = __builtin_fmaf((float)(int8_t)(w[i] >> (8 * k)), xv[4 * i + k], s[i >> 1]);
+            acc[r] = __builtin_fmaf(f16_to_f32_hw(d[r]), s[0] + s[1], acc[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float v = wave_sum(acc[r]);
+        if (lane == 0) red[wv][r] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < R && m0 + (int)threadIdx.x < M) {
+        float v = 0.f;
+        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) v += red[w][threadIdx.x];
+        y[m0 + threadIdx.x] = v;
+    }
+}
+
+// Eight rows per workgroup (x read half as often; whole lines of the TILED
+// layout); four on the row layout while eight leave a CU without two
+// workgroups.
+constexpr int Q8V_WIDE_ROWS = 8 * 512;
+
+int launch_q8_gemv(const void* W, bool tiled, int M, int K, const float* x, float* y, hipStream_t s) {
+    if (M < 1 || K < Q8_ELEMS || K % Q8_ELEMS) { set_error(-1, "q8_0 matvec: M=%d, K=%d", M, K); return -1; }
+    if ((uintptr_t)x % 16) { set_error(-1, "q8_0 matvec: the activation row must be 16-byte aligned"); return -1; }
+    const int nhalf = K / 16;
+    const int passes = (nhalf + 64 * Q8V_WAVES - 1) / (64 * Q8V_WAVES);
+    const dim3 nt(((nhalf + passes - 1) / passes + 63) / 64 * 64);
+    const uint8_t* w = (const uint8_t*)W;
+    if (tiled)
+        hipLaunchKernelGGL((q8_gemv_kernel<8, true>), dim3((M + 7) / 8), nt, 0, s, w, x, y, M, nhalf);
+    else if (M >= Q8V_WIDE_ROWS)
+        hipLaunchKernelGGL((q8_gemv_kernel<8, false>), dim3((M + 7) / 8), nt, 0, s, w, x, y, M, nhalf);
+    else
+        hipLaunchKernelGGL((q8_gemv_kernel<4, false>), dim3((M + 3) / 4), nt, 0, s, w, x, y, M, nhalf);
+    SH_CHECK_LAUNCH();
+    return 0;
 }
 
 static int cu_count() {

@@ -58,3 +58,47 @@ def test_linear_batch_special_values(hip):
     assert np.all(np.isfinite(got[[0, 2]][:, keep]))
     assert abs(got[0, 0] - want[0, 0]) <= (K + 2) * 2.0 ** -149
     np.testing.assert_allclose(got[2, keep], want[2, keep], atol=(K + 2) * EPS * float(np.abs(X[2]).sum() * 4))
+
+
+def _q8(rng, M, K):
+    """Q8_0 bytes (34-byte blocks) and the weights in float64."""
+    d = rng.uniform(1e-4, 2e-2, (M, K // 32, 1)).astype(np.float16)
+    d[rng.random(d.shape) < 0.1] *= -1
+    q = rng.integers(-128, 128, (M, K // 32, 32)).astype(np.int8)
+    raw = np.concatenate([d.view(np.uint8).reshape(M, K // 32, 2), q.view(np.uint8)], -1)
+    return np.ascontiguousarray(raw.reshape(-1)), (d.astype(np.float64) * q).reshape(M, K)
+
+
+# One row: the four / eight rows a workgroup owns and the line between them
+# (4096 rows), half blocks below a wave, 512 half blocks (K 8192) and one more
+# block (two passes).  More rows: the regrouping pass at partly filled groups
+# (K % 256), one to five groups (K 32 .. 1056), row tiles (M % 16) and blocks
+# that start on any even byte.
+@pytest.mark.parametrize("B,M,K", [(1, 1, 32), (1, 3, 64), (1, 5, 1024), (1, 4095, 96), (1, 4097, 288), (1, 9, 8192),
+                                   (1, 7, 8224), (1, 17, 14336), (2, 1, 32), (3, 15, 288), (16, 33, 224),
+                                   (17, 100, 800), (64, 47, 544), (65, 260, 1056)])
+def test_q8_row_layout_edges(hip, B, M, K):
+    rng = np.random.default_rng(B * 131 + M * 17 + K)
+    raw, w = _q8(rng, M, K)
+    X = rng.normal(0, 1, (B, K)).astype(np.float32)
+    X[0, :32] *= 1e3
+    A = DB(raw.size + 16)
+    A.upload(np.concatenate([np.zeros(2, np.uint8), raw]))   # blocks start on any even byte
+    T, R0 = DB(hip.lib.slate_hip_q8_0_tiled_bytes(M, K)), DB.from_array(raw)
+    check(hip.lib.slate_hip_q8_0_tile(T.p, R0.p, M, K), "q8_0_tile")
+    Xd, Y, Yt = DB.from_array(X), DB(B * M * 4), DB(B * M * 4)
+    check(hip.lib.slate_hip_matmul_q8_0(Y.p, A.ptr + 2, Xd.p, B, M, K), "matmul_q8_0")
+    check(hip.lib.slate_hip_matmul_q8_0_tiled(Yt.p, T.p, Xd.p, B, M, K), "matmul_q8_0_tiled")
+    got, tiled = host(Y, (B, M)), host(Yt, (B, M))
+    assert np.array_equal(got.view(np.uint32), tiled.view(np.uint32))
+    X6 = X.astype(np.float64)
+    # one row: 8 products, their sum, d, at most two passes, 6 + 8 sums: under
+    # 32 roundings of the absolute sum.  More rows: x as two f16 (2^-22 of the
+    # group's largest value each) and a rounding per MFMA, d and group sum.
+    size = np.abs(X6) @ np.abs(w).T
+    if B == 1:
+        bound = 32 * EPS * size
+    else:
+        xmax = np.repeat(np.abs(np.pad(X6, ((0, 0), (0, -K % 256)))).reshape(B, -1, 256).max(-1), 256, 1)[:, :K]
+        bound = (K // 32 * 18 + 32) * EPS * size + 2.0 ** -22 * (xmax @ np.abs(w).T)
+    assert np.all(np.abs(got - X6 @ w.T) <= bound)
