@@ -434,7 +434,7 @@ int slate_hip_rmsnorm_rows(float* y, const float* x, const float* w, int B, int 
     if (!ensure()) return -7;
     SH_REQUIRE(y && x && w && B > 0 && D > 0, "rmsnorm_rows: bad arguments");
     std::lock_guard<std::mutex> lk(g_enqueue_mu);
-    return launch_rmsnorm_rows(y, (float*)x, nullptr, 1, 0, w, B, D, eps, g_stream);
+    return launch_rmsnorm_rows(y, x, w, B, D, eps, g_stream);
 }
 
 void slate_hip_rmsnorm_row(float* y, const float* x, const float* w, int D, float eps) {
@@ -508,15 +508,34 @@ int slate_hip_rope_rows(float* x, const int32_t* pos, int n_rows, int n_heads, i
         SH_CHECK_HIP(hipMemcpy(t.dev, host.data(), host.size() * sizeof(float), hipMemcpyHostToDevice));
         t.max_pos = max_pos;
     }
-    int* bad = (int*)scratch(2, 256);
-    if (!bad) return -2;
-    SH_CHECK_HIP(hipMemsetAsync(bad, 0, sizeof(int), g_stream));
-    int rc = launch_rope_rows(x, pos, n_rows, n_heads, head_dim, t.dev, max_pos, bad, g_stream);
+    // a kernel that meets a bad row raises the flag in host memory; the count
+    // in device memory is zero between calls, so calls without bad rows need
+    // neither a clear before the kernel nor a copy after it
+    static int *bad = nullptr, *flag = nullptr, *flag_dev = nullptr;   // guarded by g_enqueue_mu
+    if (!flag_dev) {
+        if (!bad) {
+            SH_CHECK_HIP(hipMalloc(&bad, sizeof(int)));
+            const hipError_t e = hipMemsetAsync(bad, 0, sizeof(int), g_stream);
+            if (e != hipSuccess) {
+                (void)hipFree(bad);
+                bad = nullptr;
+                SH_CHECK_HIP(e);
+            }
+        }
+        if (!flag) SH_CHECK_HIP(hipHostMalloc((void**)&flag, sizeof(int)));
+        SH_CHECK_HIP(hipHostGetDevicePointer((void**)&flag_dev, flag, 0));
+    }
+    *(volatile int*)flag = 0;
+    int rc = launch_rope_rows(x, pos, n_rows, n_heads, head_dim, t.dev, max_pos, bad, flag_dev, g_stream);
     if (rc) return rc;
-    int hbad = 0;
-    SH_CHECK_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, g_stream));
     SH_CHECK_HIP(hipStreamSynchronize(g_stream));
-    SH_REQUIRE(hbad == 0, "rope_rows: %d rows with |pos| >= max_pos=%d left unrotated", hbad, max_pos);
+    if (*(volatile int*)flag) {
+        int hbad = 0;
+        SH_CHECK_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, g_stream));
+        SH_CHECK_HIP(hipMemsetAsync(bad, 0, sizeof(int), g_stream));
+        SH_CHECK_HIP(hipStreamSynchronize(g_stream));
+        SH_REQUIRE(hbad == 0, "rope_rows: %d rows with |pos| >= max_pos=%d left unrotated", hbad, max_pos);
+    }
     return 0;
 }
 

@@ -8,14 +8,13 @@
 namespace slate_hip {
 
 // k_rows.hip
-int launch_rmsnorm_rows(float* y, float* x, const float* delta, int nsplit, int64_t split_stride,
-                        const float* w, int B, int D, float eps, hipStream_t s);
+int launch_rmsnorm_rows(float* y, const float* x, const float* w, int B, int D, float eps, hipStream_t s);
 int launch_silu_mul(float* y, const float* gate, const float* up, int rows, int H, int nsplit,
                     int64_t split_stride, int64_t gate_ld, int64_t up_ld, hipStream_t s);
 int launch_add(float* y, const float* x, int64_t n, hipStream_t s);
 int launch_embed_rows(float* y, const float* W, const int32_t* tok, int T, int V, int D, hipStream_t s);
 int launch_rope_rows(float* x, const int32_t* pos, int n_rows, int n_heads, int hd, const float* cs,
-                     int max_pos, int* bad, hipStream_t s);
+                     int max_pos, int* bad, int* flag, hipStream_t s);
 // Fused engine epilogues; `a` (nullable) receives the Q4_K activation operand
 // of rows_pad rows (rows past `rows` zero), y (nullable) the f32 rows.
 int launch_rmsnorm_act(float* y, float* x, const float* delta, int nsplit, int64_t split_stride, const float* w,

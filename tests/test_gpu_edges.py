@@ -102,3 +102,43 @@ def test_q8_row_layout_edges(hip, B, M, K):
         xmax = np.repeat(np.abs(np.pad(X6, ((0, 0), (0, -K % 256)))).reshape(B, -1, 256).max(-1), 256, 1)[:, :K]
         bound = (K // 32 * 18 + 32) * EPS * size + 2.0 ** -22 * (xmax @ np.abs(w).T)
     assert np.all(np.abs(got - X6 @ w.T) <= bound)
+
+
+# Widths around the one-, two- and four-float4 forms (4096, 8192, 16384), odd
+# widths and rows that start off 16 bytes (the plain form); y may be x.
+@pytest.mark.parametrize("D,off", [(1, 0), (3, 0), (4, 0), (256, 1), (260, 0), (4096, 0), (4100, 0), (8192, 0),
+                                   (8196, 0), (12289, 0), (16384, 0), (16388, 0), (4096, 3)])
+def test_rmsnorm_rows_widths(hip, D, off):
+    rng = np.random.default_rng(D + off)
+    B, eps = 3, 1e-5
+    x = rng.normal(0, 2, (B, D)).astype(np.float32)
+    w = rng.normal(1, 0.2, D).astype(np.float32)
+    xb = DB(B * D * 4 + 32)
+    pad = np.zeros(off, np.float32)
+    xb.upload(np.concatenate([pad, x.reshape(-1), np.full(4, 9, np.float32)]))
+    y, wd = DB(B * D * 4), DB.from_array(w)
+    check(hip.rmsnorm_rows(y.p, xb.ptr + 4 * off, wd.p, B, D, eps), "rmsnorm_rows")
+    check(hip.rmsnorm_rows(xb.ptr + 4 * off, xb.ptr + 4 * off, wd.p, B, D, eps), "rmsnorm_rows in place")
+    x6 = x.astype(np.float64)
+    want = x6 * w / np.sqrt((x6 * x6).mean(-1, keepdims=True) + np.float64(np.float32(eps)))
+    raw = host(xb, (off + B * D + 4,))
+    assert np.all(raw[-4:] == 9)
+    for got in (host(y, (B, D)), raw[off:off + B * D].reshape(B, D)):
+        # at most 17 squares per thread in f32 (half of their roundings under
+        # the root), then eight roundings to the product
+        assert np.all(np.abs(got - want) <= 20 * EPS * np.abs(want))
+
+
+def test_rope_rows_counts_bad_rows_of_each_call(hip):
+    x = np.ones((6, 8), np.float32)
+    for bad in (2, 1, 0, 3, 0):
+        pos = np.array([5] * (6 - bad) + [9, -9, 8][:bad], np.int32)
+        xb = DB.from_array(x)
+        hip.lib.slate_hip_clear_error()
+        rc = hip.rope_rows(xb.p, DB.from_array(pos).p, 6, 1, 8, 10000.0, 8)
+        err = hip.lib.slate_hip_last_error()
+        hip.lib.slate_hip_clear_error()
+        assert rc == (-1 if bad else 0)
+        assert (b"%d rows" % bad in err) if bad else err is None
+        got = host(xb, (6, 8))
+        assert np.array_equal(got[6 - bad:], x[6 - bad:]) and not np.any(np.all(got[:6 - bad] == 1, -1))
