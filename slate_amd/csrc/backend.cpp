@@ -283,7 +283,7 @@ static int matmul_q4k_common(float* Y, const void* A, const float* X, int B, int
     // one row: one GEMV kernel straight into Y (no operand, no partials)
     if (B <= GEMV_ROUTE_ROWS && ((uintptr_t)X & 15) == 0)
         return launch_q4k_gemv(&t, 1, tiled, X, K, B, K, Y, M, g_stream);
-    if (B <= 16) {
+    if (B <= 16 && q4k_conv_pays(B, M, K)) {
         // one activation tile: the matmul makes its operand from X itself,
         // then the split sum (two kernels per call)
         const int max_splits = 32;
@@ -303,8 +303,9 @@ static int matmul_q4k_common(float* Y, const void* A, const float* X, int B, int
     float* part = (float*)scratch(1, (size_t)max_splits * a.rows_pad * M * sizeof(float));
     if (!part) return -2;
     int S = 1;
-    rc = launch_q4k(&t, 1, tiled, a, part, (int64_t)M, (int64_t)a.rows_pad * M, max_splits, &S, g_stream);
-    if (rc) return rc;
+    rc = launch_q4k(&t, 1, tiled, a, part, (int64_t)M, (int64_t)a.rows_pad * M, max_splits, &S, g_stream, nullptr,
+                    nullptr, Y);
+    if (rc || S == 1) return rc;                      // one split: the rows are in Y
     return launch_sum_splits(Y, part, S, B, a.rows_pad, M, g_stream);
 }
 
@@ -343,8 +344,9 @@ int slate_hip_matmul_q4k_noalloc(float* Y, const void* A, const float* X, int B,
     int rc = launch_act16_from_f32(a, X, K, g_stream);
     if (rc) return rc;
     int S = 1;
-    rc = launch_q4k(&t, 1, false, a, part, (int64_t)M, (int64_t)a.rows_pad * M, max_splits, &S, g_stream);
-    if (rc) return rc;
+    rc = launch_q4k(&t, 1, false, a, part, (int64_t)M, (int64_t)a.rows_pad * M, max_splits, &S, g_stream, nullptr,
+                    nullptr, Y);
+    if (rc || S == 1) return rc;
     return launch_sum_splits(Y, part, S, B, a.rows_pad, M, g_stream);
 }
 

@@ -429,6 +429,7 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, cons
         if (b < nb) step(w1, w0, b);
     }
     if (!active) return;
+    const bool all = tg.row_end >= 16 * NT;           // wave-uniform: partials have every padded row
     float* o = out + (int64_t)blockIdx.y * split_stride + col;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -437,7 +438,9 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, cons
 #pragma unroll
             for (int n = 0; n < NT; ++n)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[(int64_t)(16 * n + 4 * g + i) * ldo + row] = acc[r][n][i];
+                for (int i = 0; i < 4; ++i)
+                    if (all || 16 * n + 4 * g + i < tg.row_end)
+                        o[(int64_t)(16 * n + 4 * g + i) * ldo + row] = acc[r][n][i];
         }
     }
 }
@@ -763,15 +766,23 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_pf_kernel(Q4kTargets tg, const
         }
         if (!active) return;
         float* o = out + (int64_t)blockIdx.y * split_stride + col;
+        // whole tiles of rows, or (a caller's own output) up to its last row
+        auto store = [&](auto whole) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int row = (tile0 + r) * 16 + j;
-            if (tile0 + r >= tiles || row >= M) continue;
+            for (int r = 0; r < R; ++r) {
+                const int row = (tile0 + r) * 16 + j;
+                if (tile0 + r >= tiles || row >= M) continue;
 #pragma unroll
-            for (int n = 0; n < NTA; ++n)
+                for (int n = 0; n < NTA; ++n)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[(int64_t)((at0 + n) * 16 + 4 * g + i) * ldo + row] = acc[r][n][i];
-        }
+                    for (int i = 0; i < 4; ++i) {
+                        const int b = (at0 + n) * 16 + 4 * g + i;
+                        if (decltype(whole)::value || b < tg.row_end) o[(int64_t)b * ldo + row] = acc[r][n][i];
+                    }
+            }
+        };
+        if (tg.row_end >= 16 * (at0 + NTA)) store(std::true_type{});
+        else store(std::false_type{});
     };
     // nt is the same for the whole workgroup (blockIdx.z); the barriers
     // inside run() are reached by every wave of it
@@ -882,13 +893,24 @@ static int pf_slots(int NT) {
 }
 
 int launch_q4k(const Q4kTarget* t, int n, bool tiled, const Act16& a, float* out, int64_t ldo, int64_t split_stride,
-               int max_splits, int* S_out, hipStream_t s, hipEvent_t ev_start, hipEvent_t ev_stop) {
-    if (n < 1 || n > 3) { set_error(-1, "q4k: 1..3 fused tensors"); return -1; }
+               int max_splits, int* S_out, hipStream_t s, hipEvent_t ev_start, hipEvent_t ev_stop, float* direct) {
+    if (n < 1 || n > 3 || (direct && n != 1)) { set_error(-1, "q4k: 1..3 fused tensors"); return -1; }
     const int nblk = a.K / QK;
     if (nblk < 1) { set_error(-1, "q4k: K=%d", a.K); return -1; }
     if (!a.frag || a.rows_pad < 16 || a.rows_pad % 16) { set_error(-1, "q4k: bad operand buffer"); return -1; }
     if (max_splits < 1) max_splits = 1;
     const int act_tiles = a.rows_pad / 16;
+    // the whole padded rows of partials, or one split's valid rows straight
+    // into the caller's output
+    auto target = [&](Q4kTargets& tg, int S) {
+        tg.row_end = a.rows_pad;
+        if (direct && S == 1) {
+            out = direct;
+            ldo = t[0].M;
+            tg.col[0] = 0;
+            tg.row_end = a.rows;
+        }
+    };
     // up to 32 rows: the decode kernel with one or two activation tiles
     // (SLATE_HIP_Q4K_DEC32=0 sends 17..32 rows to the prompt kernel)
     if (act_tiles > 2 || (act_tiles == 2 && !knobs().q4k_dec32)) {
@@ -965,6 +987,7 @@ int launch_q4k(const Q4kTarget* t, int n, bool tiled, const Act16& a, float* out
         if (S_env > 0) S = std::min(S_env, std::max(1, std::min(max_splits, nblk)));
         const int bps = (nblk + S - 1) / S;
         S = (nblk + bps - 1) / bps;
+        target(tg, S);
         if (NT == 4) {
             if (tiled) launch_pf<4, true>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
             else launch_pf<4, false>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
@@ -993,6 +1016,7 @@ int launch_q4k(const Q4kTarget* t, int n, bool tiled, const Act16& a, float* out
     }
     tg.n = n;
     tg.grp_end = grp;
+    target(tg, S);
     if (tiled) {
         if (R == 4) launch_dec<4, true>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
         else if (R == 2) launch_dec<2, true>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
@@ -1017,6 +1041,19 @@ static void launch_dec_conv(const Q4kTargets& tg, const float* X, int64_t ldx, i
                        out, ldo, ss, nblk, bps, 0, X, ldx, rows);
 }
 
+// The CONV form saves the operand kernel's launch (about 4 us where launches
+// are what a call costs), but every workgroup converts its split's rows for
+// itself.  The operand pays where the plan on it is unsplit (then it writes
+// the final rows: two launches either way; 128256 x 4096 at 16 rows 97 -> 69
+// us, 32000 x 2048 15.9 -> 12.7), and where the matmul is long enough: from
+// 28672 x 4096 at any row count (2 rows 24.7 -> 19.7 us), at 13-16 rows from
+// 14336 x 4096 (15.9 -> 14.5 us; 4096 x 11008 15.1 -> 15.9, so not there).
+bool q4k_conv_pays(int rows, int M, int K) {
+    int tiles = (M + 15) / 16, R, S;
+    dec_plan(&tiles, 1, K / QK, 32, DEC_BPS_STEP, &R, &S);
+    return S > 1 && (double)M * K < (rows > 12 ? 50.0 : 80.0) * 1048576.0;
+}
+
 int launch_q4k_conv(const Q4kTarget& t, bool tiled, const float* X, int64_t ldx, int rows, int K, float* out,
                     int64_t ldo, int64_t split_stride, int max_splits, int* S_out, hipStream_t s) {
     const int nblk = K / QK;
@@ -1037,6 +1074,7 @@ int launch_q4k_conv(const Q4kTarget& t, bool tiled, const float* X, int64_t ldx,
     tg.grp0[0] = 0;
     tg.n = 1;
     tg.grp_end = (tiles + R - 1) / R;
+    tg.row_end = 16;
     if (tiled) {
         if (R == 4) launch_dec_conv<4, true>(tg, X, ldx, rows, out, ldo, split_stride, nblk, bps, S, s);
         else if (R == 2) launch_dec_conv<2, true>(tg, X, ldx, rows, out, ldo, split_stride, nblk, bps, S, s);

@@ -142,3 +142,53 @@ def test_rope_rows_counts_bad_rows_of_each_call(hip):
         assert (b"%d rows" % bad in err) if bad else err is None
         got = host(xb, (6, 8))
         assert np.array_equal(got[6 - bad:], x[6 - bad:]) and not np.any(np.all(got[:6 - bad] == 1, -1))
+
+
+def _q4k(rng, M, K):
+    """Q4_K bytes, the weights in float64 and the size of their two terms
+    (d sc q and dmin mn)."""
+    raw = rng.integers(0, 256, (M * K // 256, 144), dtype=np.uint8)
+    head = rng.uniform(1e-5, 1e-3, (raw.shape[0], 2)).astype(np.float16)
+    raw[:, :4] = head.view(np.uint8).reshape(-1, 4)
+    s = raw[:, 4:16].astype(np.int64)
+    sc = np.concatenate([s[:, 0:4] & 63, (s[:, 8:12] & 15) | (s[:, 0:4] >> 6 << 4)], 1)
+    mn = np.concatenate([s[:, 4:8] & 63, (s[:, 8:12] >> 4) | (s[:, 4:8] >> 6 << 4)], 1)
+    q = raw[:, 16:].reshape(-1, 8, 16)
+    q = np.concatenate([q & 15, q >> 4], 2).astype(np.float64)
+    a = (head[:, 0:1].astype(np.float64) * sc)[..., None] * q
+    b = (head[:, 1:2].astype(np.float64) * mn)[..., None] * np.ones(32)
+    return raw.reshape(-1), (a - b).reshape(M, K), (a + b).reshape(M, K)
+
+
+# Unsplit plans write the caller's rows themselves: row counts inside and at
+# the end of 16-row tiles on the decode kernel (one and two tiles) and the
+# prompt kernel (groups of two and four tiles and a shorter last one); and
+# the line between the two forms for at most 16 rows (8000 x 256: split).
+@pytest.mark.parametrize("B,M,K", [(2, 49163, 256), (13, 49163, 256), (16, 50001, 512), (17, 49163, 256),
+                                   (32, 49163, 256), (33, 40007, 512), (63, 40007, 256), (65, 40007, 256),
+                                   (9, 8000, 512), (13, 3000, 19968)])
+@pytest.mark.parametrize("form", ["row", "tiled", "noalloc"])
+def test_q4k_rows_of_the_output(hip, B, M, K, form):
+    if form == "noalloc" and B * M > 1.5e6:
+        pytest.skip("one split of partials is over that entry's fixed scratch")
+    rng = np.random.default_rng(B + M + K)
+    raw, w, size = _q4k(rng, M, K)
+    X = rng.normal(0, 1, (B, K)).astype(np.float32)
+    A, Xd, Y = DB.from_array(raw), DB.from_array(X), DB((B * M + 64) * 4)
+    Y.upload(np.full(B * M + 64, 7.0, np.float32))
+    if form == "tiled":
+        T = DB(hip.lib.slate_hip_q4k_tiled_bytes(M, K))
+        check(hip.lib.slate_hip_q4k_tile(T.p, A.p, M, K), "q4k_tile")
+        check(hip.lib.slate_hip_matmul_q4k_tiled(Y.p, T.p, Xd.p, B, M, K), "matmul_q4k_tiled")
+    elif form == "row":
+        check(hip.matmul_q4k(Y.p, A.p, Xd.p, B, M, K), "matmul_q4k")
+    else:
+        check(hip.lib.slate_hip_matmul_q4k_noalloc(Y.p, A.p, Xd.p, B, M, K), "matmul_q4k_noalloc")
+    got = host(Y, (B * M + 64,))
+    assert np.all(got[B * M:] == 7.0)
+    X6 = X.astype(np.float64)
+    # x and its sub-block sums as two f16 (2^-22 of the block's largest value,
+    # 32 of them to a sum), then at most 24 roundings per 256-element block
+    xmax = np.repeat(np.abs(X6).reshape(B, -1, 256).max(-1), 256, 1)
+    bound = (K // 256 * 24 + 32) * EPS * (np.abs(X6) @ size.T) + 2.0 ** -21 * (xmax @ size.T)
+    assert np.all(np.abs(got[:B * M].reshape(B, M) - X6 @ w.T) <= bound)
