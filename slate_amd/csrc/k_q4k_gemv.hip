@@ -30,6 +30,7 @@
 namespace slate_hip {
 
 constexpr int GEMV_WAVES = 8;                  // 512 threads
+constexpr int GEMV_XPITCH = 36;                // floats of LDS per thread's 32 of x (16-byte reads without conflicts)
 
 // x & m in inline assembly: the compiler cannot fold the mask into the byte
 // extractions that follow, so each masked byte becomes a float with one
@@ -44,11 +45,17 @@ __device__ __forceinline__ uint32_t and_opaque(uint32_t x, uint32_t m) {
 // tg: up to three tensors sharing X; tensor i owns workgroups
 // [grp0[i], grp0[i+1]) of R rows each and writes Y columns [col, col + M).
 // X: nb rows (nb <= B) of K f32, ldx apart; Y: nb rows, ldy apart.
-template <int B, int R, bool TILED>
+// XLDS (one row): a thread's 32 values of x are 128 bytes apart from the next
+// thread's, so loading them directly touches 64 lines per load, eight times
+// over; the wave instead loads its 8 KiB line by line and hands them out
+// through LDS (4096 x 4096 5.64 -> 5.34 us per call, 4096 x 14336 11.8 ->
+// 11.1, 128256 x 4096 67 -> 64.6; 1024 x 1024 4.1 -> 4.3, so not there).
+template <int B, int R, bool TILED, bool XLDS>
 __global__ __launch_bounds__(64 * GEMV_WAVES) void q4k_gemv_kernel(Q4kTargets tg, const float* __restrict__ X,
                                                                    int64_t ldx, int nb, float* __restrict__ Y,
                                                                    int64_t ldy, int nblk) {
     __shared__ float red[GEMV_WAVES * 4 * R * B];
+    extern __shared__ __align__(16) float s_x[];      // XLDS: 64 x GEMV_XPITCH floats a wave
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wv = t >> 6;
@@ -75,17 +82,14 @@ __global__ __launch_bounds__(64 * GEMV_WAVES) void q4k_gemv_kernel(Q4kTargets tg
         const int kb = kc + (t >> 3);
         const bool live = kb < nblk;
         const int kbc = live ? kb : nblk - 1;
-        float x[B][32], xs[B];
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-            const float4* xp = (const float4*)(X + (int64_t)min(b, nb - 1) * ldx + (int64_t)kbc * QK + 32 * s);
+        // XLDS: the wave's 64 x 32 values by whole lines, before the weights
+        float4 v[XLDS ? 8 : 1];
+        if constexpr (XLDS) {
+            const int64_t e0 = (int64_t)kc * QK + wv * 2048;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float4 v = (b < nb && live) ? xp[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-                x[b][4 * i] = v.x;
-                x[b][4 * i + 1] = v.y;
-                x[b][4 * i + 2] = v.z;
-                x[b][4 * i + 3] = v.w;
+                const int64_t e = e0 + 4 * (64 * i + lane);
+                v[i] = e < (int64_t)nblk * QK ? *(const float4*)(X + e) : make_float4(0.f, 0.f, 0.f, 0.f);
             }
         }
         uint4 hd[R], qv[R];
@@ -104,6 +108,38 @@ __global__ __launch_bounds__(64 * GEMV_WAVES) void q4k_gemv_kernel(Q4kTargets tg
             }
             hd[r] = *(const uint4*)hp;
             qv[r] = *(const uint4*)qp;
+        }
+        float x[B][32], xs[B];
+        if constexpr (XLDS) {
+            // handed out through LDS (a wave's own slice: no barrier)
+            float* sx = s_x + wv * 64 * GEMV_XPITCH;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int f = 64 * i + lane;
+                *(float4*)(sx + (f >> 3) * GEMV_XPITCH + 4 * (f & 7)) = v[i];
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float4 q = *(const float4*)(sx + lane * GEMV_XPITCH + 4 * i);
+                x[0][4 * i] = q.x;
+                x[0][4 * i + 1] = q.y;
+                x[0][4 * i + 2] = q.z;
+                x[0][4 * i + 3] = q.w;
+            }
+            __builtin_amdgcn_wave_barrier();
+        } else
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const float4* xp = (const float4*)(X + (int64_t)min(b, nb - 1) * ldx + (int64_t)kbc * QK + 32 * s);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float4 v = (b < nb && live) ? xp[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+                x[b][4 * i] = v.x;
+                x[b][4 * i + 1] = v.y;
+                x[b][4 * i + 2] = v.z;
+                x[b][4 * i + 3] = v.w;
+            }
         }
 #pragma unroll
         for (int b = 0; b < B; ++b) {
@@ -158,14 +194,17 @@ __global__ __launch_bounds__(64 * GEMV_WAVES) void q4k_gemv_kernel(Q4kTargets tg
     }
 }
 
-template <int B, int R>
+static size_t gemv_x_bytes(int nw) { return (size_t)nw * 64 * GEMV_XPITCH * sizeof(float); }
+
+template <int B, int R, bool XLDS>
 static void launch_gemv(const Q4kTargets& tg, bool tiled, const float* X, int64_t ldx, int nb, float* Y,
                         int64_t ldy, int nblk, int nw, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+    const size_t lds = XLDS ? gemv_x_bytes(nw) : 0;
     if (tiled)
-        SH_LAUNCH(e0, e1, (q4k_gemv_kernel<B, R, true>), dim3(tg.grp_end), dim3(64 * nw), 0, s, tg, X, ldx, nb, Y,
+        SH_LAUNCH(e0, e1, (q4k_gemv_kernel<B, R, true, XLDS>), dim3(tg.grp_end), dim3(64 * nw), lds, s, tg, X, ldx, nb, Y,
                   ldy, nblk);
     else
-        SH_LAUNCH(e0, e1, (q4k_gemv_kernel<B, R, false>), dim3(tg.grp_end), dim3(64 * nw), 0, s, tg, X, ldx, nb, Y,
+        SH_LAUNCH(e0, e1, (q4k_gemv_kernel<B, R, false, XLDS>), dim3(tg.grp_end), dim3(64 * nw), lds, s, tg, X, ldx, nb, Y,
                   ldy, nblk);
 }
 
@@ -202,12 +241,16 @@ int launch_q4k_gemv(const Q4kTarget* t, int n, bool tiled, const float* X, int64
     tg.n = n;
     tg.grp_end = grp;
     const int nw = std::min(GEMV_WAVES, (nblk + 7) / 8);
+    // below about 6M weights a call costs its launch and the kernel's latency
+    const bool xlds = (double)grp * R * K >= 6.0 * 1048576.0;
     if (r16)
-        SH_LAUNCH(ev_start, ev_stop, (q4k_gemv_kernel<1, 16, false>), dim3(tg.grp_end), dim3(64 * nw), 0, s, tg, X,
+        SH_LAUNCH(ev_start, ev_stop, (q4k_gemv_kernel<1, 16, false, true>), dim3(tg.grp_end), dim3(64 * nw),
+                  gemv_x_bytes(nw), s, tg, X,
                   ldx, B, Y, ldy, nblk);
-    else if (B == 1) launch_gemv<1, 8>(tg, tiled, X, ldx, B, Y, ldy, nblk, nw, s, ev_start, ev_stop);
-    else if (B == 2) launch_gemv<2, 8>(tg, tiled, X, ldx, B, Y, ldy, nblk, nw, s, ev_start, ev_stop);
-    else launch_gemv<4, 4>(tg, tiled, X, ldx, B, Y, ldy, nblk, nw, s, ev_start, ev_stop);
+    else if (B == 1 && xlds) launch_gemv<1, 8, true>(tg, tiled, X, ldx, B, Y, ldy, nblk, nw, s, ev_start, ev_stop);
+    else if (B == 1) launch_gemv<1, 8, false>(tg, tiled, X, ldx, B, Y, ldy, nblk, nw, s, ev_start, ev_stop);
+    else if (B == 2) launch_gemv<2, 8, false>(tg, tiled, X, ldx, B, Y, ldy, nblk, nw, s, ev_start, ev_stop);
+    else launch_gemv<4, 4, false>(tg, tiled, X, ldx, B, Y, ldy, nblk, nw, s, ev_start, ev_stop);
     SH_CHECK_LAUNCH();
     return 0;
 }

@@ -192,3 +192,24 @@ def test_q4k_rows_of_the_output(hip, B, M, K, form):
     xmax = np.repeat(np.abs(X6).reshape(B, -1, 256).max(-1), 256, 1)
     bound = (K // 256 * 24 + 32) * EPS * (np.abs(X6) @ size.T) + 2.0 ** -21 * (xmax @ size.T)
     assert np.all(np.abs(got[:B * M].reshape(B, M) - X6 @ w.T) <= bound)
+
+
+# One row: x handed out through LDS (from 6M weights on) and loaded directly,
+# with whole and partly filled waves of blocks, one and two passes over K, and
+# the 16-row workgroups of long rows.
+@pytest.mark.parametrize("M,K", [(1535, 4096), (1537, 4096), (6145, 1024), (6143, 1024), (3001, 2304), (455, 14336),
+                                 (330, 19968), (25000, 256)])
+def test_q4k_matvec_activation_paths(hip, M, K):
+    rng = np.random.default_rng(M + K)
+    raw, w, size = _q4k(rng, M, K)
+    x = rng.normal(0, 1, K).astype(np.float32)
+    y = DB((M + 16) * 4)
+    y.upload(np.full(M + 16, 7.0, np.float32))
+    hip.matvec_q4k(y.p, DB.from_array(raw).p, DB.from_array(x).p, M, K)
+    check(0, "matvec_q4k")
+    got = host(y, (M + 16,))
+    assert np.all(got[M:] == 7.0)
+    # per sub-block 16 products twice and the sum of 32 x, their scales, then
+    # up to three passes, 4 + 32 sums: under 80 roundings of the absolute sum
+    x6 = x.astype(np.float64)
+    assert np.all(np.abs(got[:M] - w @ x6) <= 80 * EPS * (size @ np.abs(x6)))
