@@ -131,6 +131,7 @@ struct RowNorm {
     const float* ssq;
     int nblk, D;
     float eps;
+    const float* inv = nullptr;     // the rows' factors, where a kernel computed them once (prompt steps)
 };
 
 // Up to three Q4_K tensors sharing one input, fused into one launch; tensor i

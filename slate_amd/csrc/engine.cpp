@@ -79,6 +79,7 @@ struct slate_hip_llama {
     float* part = nullptr;
     size_t part_floats = 0;
     float* ssq = nullptr;          // [T_pad][D/256] block sums of squares (deferred RMSNorm)
+    float* inv = nullptr;          // [T_pad] row factors from them (prompt steps)
     bool defer_norm = true;
     bool tokenwise_attn = false;   // prompt-chunk tokens through the decode attention kernel
     bool prompt_mfma = false;      // prompt-chunk blocks may go to the MFMA prompt attention kernel
@@ -228,7 +229,7 @@ int alloc_runtime(slate_hip_llama* m) {
     char* fr = nullptr;
     if (dalloc(m, &fr, act_frag_bytes((int)T, Kmax))) return -2;
     m->act = Act16{fr, 0, (int)T, Kmax};
-    if (dalloc(m, &m->ssq, T * (D / QK + 1))) return -2;
+    if (dalloc(m, &m->ssq, T * (D / QK + 1)) || dalloc(m, &m->inv, T)) return -2;
     m->defer_norm = getenv("SLATE_HIP_FUSED_NORM") == nullptr || atoi(getenv("SLATE_HIP_FUSED_NORM")) != 0;
     // opt-in: at 8B shapes a decode step is not launch-bound (graph replay
     // measured 3.37 ms per B=16 step against 3.35 ms launched eagerly)
@@ -446,6 +447,16 @@ bool defer_norm(const slate_hip_llama* m, const GroupIn& gi, int D) {
     return m->defer_norm && gi.q4 && !gi.rows() && D % QK == 0;
 }
 
+// The deferred factors of a prompt step's rows, once for all their consumers
+// (below ROW_INV_ROWS rows the extra launch costs what it saves).
+constexpr int ROW_INV_ROWS = 128;
+int norm_factors(slate_hip_llama* m, RowNorm& rn, int T, hipStream_t s) {
+    if (!rn.ssq || T < ROW_INV_ROWS || m->step_one_each) return 0;
+    const int rc = launch_row_inv(m->inv, rn, T, s);
+    if (rc == 0) rn.inv = m->inv;
+    return rc;
+}
+
 // One matmul group: the linears in `lins` read the same input (operand `a`
 // for Q4_K, rows X [T, K] for f32 and Q8_0) and write column ranges of one
 // partial buffer [S][T_pad][ldo]; *S_out = S.  Q8_0 linears write the split
@@ -586,7 +597,7 @@ int enqueue_step(slate_hip_llama* m, int n, int T, bool want_logits, hipStream_t
                 rc = launch_rmsnorm_act(gi.rows() ? m->xn : nullptr, m->x, li ? m->part : nullptr, S_prev,
                                         (int64_t)tpad * D, Ld.attn_norm, T, D, c.rms_eps, gi.q4 ? &a : nullptr, s);
             }
-            if (rc) return rc;
+            if (rc || (rc = norm_factors(m, rn, T, s))) return rc;
             if ((rc = mm_group(m, &a, m->xn, T, D, g, col, 3, D + 2 * kvd, &S, s))) return rc;
         }
         char* Kl = (char*)m->Kpool + (int64_t)li * m->layer_stride * m->kv_bytes;
@@ -641,7 +652,7 @@ int enqueue_step(slate_hip_llama* m, int n, int T, bool want_logits, hipStream_t
                 rc = launch_rmsnorm_act(gi.rows() ? m->xn : nullptr, m->x, m->part, S, (int64_t)tpad * D, Ld.ffn_norm,
                                         T, D, c.rms_eps, gi.q4 ? &a : nullptr, s);
             }
-            if (rc) return rc;
+            if (rc || (rc = norm_factors(m, rn, T, s))) return rc;
             if ((rc = mm_group(m, &a, m->xn, T, D, g, col, 2, 2 * H, &S, s))) return rc;
         }
         {
@@ -670,11 +681,10 @@ int enqueue_step(slate_hip_llama* m, int n, int T, bool want_logits, hipStream_t
         const RowNorm rl{m->ssq, D / QK, D, c.rms_eps};
         if ((rc = launch_argmax_rows(m->next, m->logits, n, c.vocab, m->argmax_ws, s, &rl))) return rc;
     } else {
-        if ((rc = launch_rmsnorm_act(m->xn, m->x, m->part, S_prev, (int64_t)tpad * D, m->out_norm, T, D,
-                                     c.rms_eps, nullptr, s)))
+        // only the rows of each sequence's last token go on to the LM head
+        if ((rc = launch_rmsnorm_act(m->xlast, m->x, m->part, S_prev, (int64_t)tpad * D, m->out_norm, n, D,
+                                     c.rms_eps, nullptr, s, m->last_tok, T)))
             return rc;
-        // rows of each sequence's last token -> xlast (gather by last_tok)
-        if ((rc = launch_embed_rows(m->xlast, m->xn, m->last_tok, n, T, D, s))) return rc;
         if ((rc = lm_head(m, n, s))) return rc;
         if ((rc = launch_argmax_rows(m->next, m->logits, n, c.vocab, m->argmax_ws, s))) return rc;
     }

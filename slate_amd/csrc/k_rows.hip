@@ -134,19 +134,23 @@ int launch_add(float* y, const float* x, int64_t n, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // Embedding gather: y[t, :] = W[tok[t], :].  Tokens are validated on the
 // host; out-of-range ids are clamped here only to keep every access in bounds.
-__global__ void embed_rows_kernel(float* __restrict__ y, const float* __restrict__ W,
-                                  const int32_t* __restrict__ tok, int V, int D) {
-    int t = blockIdx.y;
+template <typename V>
+__global__ __launch_bounds__(256) void embed_rows_kernel(V* __restrict__ y, const V* __restrict__ W,
+                                                         const int32_t* __restrict__ tok, int vocab, int D) {
+    const int t = blockIdx.y;
     int id = tok[t];
-    id = id < 0 ? 0 : (id >= V ? V - 1 : id);
+    id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
     for (int d = blockIdx.x * blockDim.x + threadIdx.x; d < D; d += gridDim.x * blockDim.x)
         y[(size_t)t * D + d] = W[(size_t)id * D + d];
 }
 
 int launch_embed_rows(float* y, const float* W, const int32_t* tok, int T, int V, int D, hipStream_t s) {
     if (T <= 0) return 0;
-    dim3 grid((D + 255) / 256, T);
-    hipLaunchKernelGGL(embed_rows_kernel, grid, dim3(256), 0, s, y, W, tok, V, D);
+    if (D % 4 == 0 && (((uintptr_t)y | (uintptr_t)W) & 15) == 0)
+        hipLaunchKernelGGL(embed_rows_kernel<float4>, dim3((D / 4 + 255) / 256, T), dim3(256), 0, s, (float4*)y,
+                           (const float4*)W, tok, V, D / 4);
+    else
+        hipLaunchKernelGGL(embed_rows_kernel<float>, dim3((D + 255) / 256, T), dim3(256), 0, s, y, W, tok, V, D);
     SH_CHECK_LAUNCH();
     return 0;
 }
@@ -310,16 +314,20 @@ int launch_residual_act(float* x, const float* delta, int nsplit, int64_t split_
 // (act != 0, D % 256 == 0).  One workgroup per row keeps the row in
 // registers: thread i owns elements 4(i + nt*c) .. +3 of chunk c, so each
 // wave owns whole 256-element blocks.  Rows >= rows write zero operand rows.
+// With `pick`, output row i is source row pick[i] (clamped to the src_rows
+// rows of x and delta) and x stays as it is.
 constexpr int RMS_MAX_CHUNKS = 4;
 __global__ __launch_bounds__(1024) void rmsnorm_act_kernel(float* __restrict__ y, float* __restrict__ x,
                                                            const float* __restrict__ delta, int nsplit,
                                                            int64_t split_stride, const float* __restrict__ w,
-                                                           int rows, int D, float eps, Act16 a, int act) {
+                                                           int rows, int D, float eps, Act16 a, int act,
+                                                           const int32_t* __restrict__ pick, int src_rows) {
 #pragma clang fp contract(off)
     __shared__ double sh[16];
-    const int r = blockIdx.x;
+    const int ro = blockIdx.x;                        // output row
+    const int r = pick ? min(max(pick[ro], 0), src_rows - 1) : ro;
     const int nt = blockDim.x, tid = threadIdx.x, lane = tid & 63;
-    const bool valid = r < rows;
+    const bool valid = ro < rows;
     // every load (x, w, the first eight partials of each chunk) is issued
     // before any arithmetic; x is written back after the row reduction
     float4 v[RMS_MAX_CHUNKS], wv[RMS_MAX_CHUNKS];
@@ -365,17 +373,17 @@ __global__ __launch_bounds__(1024) void rmsnorm_act_kernel(float* __restrict__ y
         if (e >= D) break;                        // uniform per wave when D % 256 == 0
         float4 yv = make_float4(0.f, 0.f, 0.f, 0.f);
         if (valid) {
-            if (delta) *(float4*)(x + (size_t)r * D + e) = v[c];
+            if (delta && !pick) *(float4*)(x + (size_t)r * D + e) = v[c];
             yv = make_float4((v[c].x * wv[c].x) * inv, (v[c].y * wv[c].y) * inv, (v[c].z * wv[c].z) * inv,
                              (v[c].w * wv[c].w) * inv);
-            if (y) *(float4*)(y + (size_t)r * D + e) = yv;
+            if (y) *(float4*)(y + (size_t)ro * D + e) = yv;
         }
-        if (act) act16_store_block(a, r, e / QK, lane, yv);
+        if (act) act16_store_block(a, ro, e / QK, lane, yv);
     }
 }
 
 int launch_rmsnorm_act(float* y, float* x, const float* delta, int nsplit, int64_t split_stride, const float* w,
-                       int rows, int D, float eps, const Act16* a, hipStream_t s) {
+                       int rows, int D, float eps, const Act16* a, hipStream_t s, const int32_t* pick, int src_rows) {
     if (rows <= 0) return 0;
     if (D % 4 || D > 4 * 1024 * RMS_MAX_CHUNKS || (a && (D % QK || a->K != D))) {
         set_error(-1, "rmsnorm_act: unsupported width %d", D);
@@ -387,7 +395,7 @@ int launch_rmsnorm_act(float* y, float* x, const float* delta, int nsplit, int64
     if (nt < 64) nt = 64;
     const int grid = a ? a->rows_pad : rows;
     hipLaunchKernelGGL(rmsnorm_act_kernel, dim3(grid), dim3(nt), 0, s, y, x, delta, nsplit, split_stride, w, rows,
-                       D, eps, a ? *a : Act16{}, a ? 1 : 0);
+                       D, eps, a ? *a : Act16{}, a ? 1 : 0, pick, src_rows);
     SH_CHECK_LAUNCH();
     return 0;
 }
@@ -400,7 +408,7 @@ int launch_rmsnorm_act(float* y, float* x, const float* delta, int nsplit, int64
 // tile), wave w = row w of the half, the operand written by
 // act16_store_tile (half tiles: at 114 VGPRs two such workgroups share a
 // CU, where one 16-row workgroup would hold it alone).
-template <int NPRE, bool TILE>
+template <int NPRE, bool TILE, bool INV>
 __device__ __forceinline__ void silu_act_body(float* __restrict__ y, const float* __restrict__ gate,
                                               const float* __restrict__ up, int rows, int H, int nsplit,
                                               int64_t split_stride, int64_t ld, const Act16& a, int act,
@@ -418,10 +426,12 @@ __device__ __forceinline__ void silu_act_body(float* __restrict__ y, const float
         const Split4N<NPRE> pg = split_load4<NPRE>(gp, nsplit, split_stride);
         const Split4N<NPRE> pu = split_load4<NPRE>(upp, nsplit, split_stride);
         RmsPre rp;
-        if (rn.ssq) rp = row_rms_load(rn.ssq, r, rn.nblk);
+        float inv = 0.f;
+        if constexpr (INV) inv = rn.inv[r];
+        else if (rn.ssq) rp = row_rms_load(rn.ssq, r, rn.nblk);
         float4 g = split_fin4(pg, gp, nsplit, split_stride), u = split_fin4(pu, upp, nsplit, split_stride);
         if (rn.ssq) {   // gate and up are linear in the normalised row
-            const float inv = row_rms_fin(rp, rn.ssq, r, rn.nblk, rn.D, rn.eps);
+            if constexpr (!INV) inv = row_rms_fin(rp, rn.ssq, r, rn.nblk, rn.D, rn.eps);
             g = make_float4(g.x * inv, g.y * inv, g.z * inv, g.w * inv);
             u = make_float4(u.x * inv, u.y * inv, u.z * inv, u.w * inv);
         }
@@ -432,19 +442,20 @@ __device__ __forceinline__ void silu_act_body(float* __restrict__ y, const float
     if constexpr (TILE) act16_store_tile<8>(a, blockIdx.y >> 1, blockIdx.y & 1, kb, s_t, h);
     else if (act) act16_store_block(a, r, kb, lane, h);
 }
-template <int NPRE>
+template <int NPRE, bool INV>
 __global__ __launch_bounds__(256) void silu_act_kernel(float* __restrict__ y, const float* __restrict__ gate,
                                                        const float* __restrict__ up, int rows, int H, int nsplit,
                                                        int64_t split_stride, int64_t ld, Act16 a, int act,
                                                        RowNorm rn) {
-    silu_act_body<NPRE, false>(y, gate, up, rows, H, nsplit, split_stride, ld, a, act, rn, nullptr);
+    silu_act_body<NPRE, false, INV>(y, gate, up, rows, H, nsplit, split_stride, ld, a, act, rn, nullptr);
 }
+template <bool INV>
 __global__ __launch_bounds__(512) void silu_act_tile_kernel(float* __restrict__ y, const float* __restrict__ gate,
                                                              const float* __restrict__ up, int rows, int H,
                                                              int nsplit, int64_t split_stride, int64_t ld, Act16 a,
                                                              RowNorm rn) {
     __shared__ uint4 s_t[ACT_FRAG_UNITS];
-    silu_act_body<1, true>(y, gate, up, rows, H, nsplit, split_stride, ld, a, 1, rn, s_t);
+    silu_act_body<1, true, INV>(y, gate, up, rows, H, nsplit, split_stride, ld, a, 1, rn, s_t);
 }
 
 int launch_silu_act(float* y, const float* gate, const float* up, int rows, int H, int nsplit,
@@ -461,15 +472,50 @@ int launch_silu_act(float* y, const float* gate, const float* up, int rows, int 
     // unsplit gate+up (prompt steps): registers for one partial each, so
     // more waves per SIMD on the prompt rows' large grids; with the operand,
     // written by 8-row half tiles
-    if (nsplit <= 1 && a && a->rows_pad > 16)
-        hipLaunchKernelGGL(silu_act_tile_kernel, dim3(nblk, a->rows_pad / 8), dim3(512), 0, s, y, gate, up, rows,
-                           H, nsplit, split_stride, ld, *a, rn);
-    else if (nsplit <= 1)
-        hipLaunchKernelGGL(silu_act_kernel<1>, grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit, split_stride,
-                           ld, a ? *a : Act16{}, a ? 1 : 0, rn);
-    else
-        hipLaunchKernelGGL(silu_act_kernel<8>, grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit, split_stride,
-                           ld, a ? *a : Act16{}, a ? 1 : 0, rn);
+    const Act16 ao = a ? *a : Act16{};
+    const int act = a ? 1 : 0;
+    if (nsplit <= 1 && a && a->rows_pad > 16) {
+        const dim3 tg(nblk, a->rows_pad / 8);
+        if (rn.inv)
+            hipLaunchKernelGGL(silu_act_tile_kernel<true>, tg, dim3(512), 0, s, y, gate, up, rows, H, nsplit,
+                               split_stride, ld, ao, rn);
+        else
+            hipLaunchKernelGGL(silu_act_tile_kernel<false>, tg, dim3(512), 0, s, y, gate, up, rows, H, nsplit,
+                               split_stride, ld, ao, rn);
+    } else if (nsplit <= 1) {
+        if (rn.inv)
+            hipLaunchKernelGGL((silu_act_kernel<1, true>), grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit,
+                               split_stride, ld, ao, act, rn);
+        else
+            hipLaunchKernelGGL((silu_act_kernel<1, false>), grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit,
+                               split_stride, ld, ao, act, rn);
+    } else if (rn.inv) {
+        hipLaunchKernelGGL((silu_act_kernel<8, true>), grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit,
+                           split_stride, ld, ao, act, rn);
+    } else {
+        hipLaunchKernelGGL((silu_act_kernel<8, false>), grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit,
+                           split_stride, ld, ao, act, rn);
+    }
+    SH_CHECK_LAUNCH();
+    return 0;
+}
+
+// The rows' RMSNorm factors from their block sums, one thread per row (the
+// same additions in the same order as the consumers' own).  In prompt steps
+// every wave of the QKV and SwiGLU epilogues otherwise repeats its row's
+// sums, in double: 48 heads and 56 blocks a row at the 8B shape (1995 rows:
+// SwiGLU 102 -> 69 us, QKV epilogue 61 -> 28 us with one load per unsplit
+// partial; this kernel 4.7 us).
+__global__ __launch_bounds__(64) void row_inv_kernel(float* __restrict__ inv, RowNorm rn, int rows) {
+    const int r = blockIdx.x * 64 + threadIdx.x;
+    if (r >= rows) return;
+    const RmsPre rp = row_rms_load(rn.ssq, r, rn.nblk);
+    inv[r] = row_rms_fin(rp, rn.ssq, r, rn.nblk, rn.D, rn.eps);
+}
+
+int launch_row_inv(float* inv, const RowNorm& rn, int rows, hipStream_t s) {
+    if (rows <= 0) return 0;
+    hipLaunchKernelGGL(row_inv_kernel, dim3((rows + 63) / 64), dim3(64), 0, s, inv, rn, rows);
     SH_CHECK_LAUNCH();
     return 0;
 }
@@ -478,7 +524,7 @@ int launch_silu_act(float* y, const float* gate, const float* up, int rows, int 
 // workgroup: sums the split-K partials of the head's columns, rotates q / k
 // at the token's position (same table and expressions as rope_apply) and
 // writes q to qout, k and v into the KV pool.
-template <typename KVT>
+template <typename KVT, int NPRE>
 __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qout, KVT* __restrict__ Kpool,
                                                      KVT* __restrict__ Vpool, const float* __restrict__ part,
                                                      int nsplit, int64_t split_stride, int qkv_ld,
@@ -500,17 +546,18 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qout, 
     // partials of the lane's columns, the row's block sums) is issued before
     // the position-dependent ones (rotation table, KV row).
     RmsPre rp;
-    if (rn.ssq) rp = row_rms_load(rn.ssq, t, rn.nblk);
     float inv = 1.0f;
+    if (rn.inv) inv = rn.inv[t];
+    else if (rn.ssq) rp = row_rms_load(rn.ssq, t, rn.nblk);
     auto scale = [&](float v) { return rn.ssq ? v * inv : v; };
     if (u < n_heads) {
         for (int i = lane; i < half; i += 64) {
             const int c0 = u * hd + i;
-            const Split1 pa = split_load1(pr + c0, nsplit, split_stride);
-            const Split1 pb = split_load1(pr + c0 + half, nsplit, split_stride);
+            const Split1N<NPRE> pa = split_load1<NPRE>(pr + c0, nsplit, split_stride);
+            const Split1N<NPRE> pb = split_load1<NPRE>(pr + c0 + half, nsplit, split_stride);
             const float c = cs[((size_t)ap * half + i) * 2 + 0];
             const float sn = sg * cs[((size_t)ap * half + i) * 2 + 1];
-            if (rn.ssq) inv = row_rms_fin(rp, rn.ssq, t, rn.nblk, rn.D, rn.eps);
+            if (rn.ssq && !rn.inv) inv = row_rms_fin(rp, rn.ssq, t, rn.nblk, rn.D, rn.eps);
             const float a = scale(split_fin1(pa, pr + c0, nsplit, split_stride));
             const float b = scale(split_fin1(pb, pr + c0 + half, nsplit, split_stride));
             qout[(size_t)t * D + c0] = a * c - b * sn;
@@ -521,14 +568,14 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qout, 
         const int seq = tok2seq[t];
         for (int i = lane; i < half; i += 64) {
             const int ck = D + kh * hd + i, cv = D + kvd + kh * hd + i;
-            const Split1 pa = split_load1(pr + ck, nsplit, split_stride);
-            const Split1 pb = split_load1(pr + ck + half, nsplit, split_stride);
-            const Split1 pv0 = split_load1(pr + cv, nsplit, split_stride);
-            const Split1 pv1 = split_load1(pr + cv + half, nsplit, split_stride);
+            const Split1N<NPRE> pa = split_load1<NPRE>(pr + ck, nsplit, split_stride);
+            const Split1N<NPRE> pb = split_load1<NPRE>(pr + ck + half, nsplit, split_stride);
+            const Split1N<NPRE> pv0 = split_load1<NPRE>(pr + cv, nsplit, split_stride);
+            const Split1N<NPRE> pv1 = split_load1<NPRE>(pr + cv + half, nsplit, split_stride);
             const float c = cs[((size_t)ap * half + i) * 2 + 0];
             const float sn = sg * cs[((size_t)ap * half + i) * 2 + 1];
             const int64_t base = kv_base[seq] + (int64_t)kh * head_stride + (int64_t)p * hd;
-            if (rn.ssq) inv = row_rms_fin(rp, rn.ssq, t, rn.nblk, rn.D, rn.eps);
+            if (rn.ssq && !rn.inv) inv = row_rms_fin(rp, rn.ssq, t, rn.nblk, rn.D, rn.eps);
             const float a = scale(split_fin1(pa, pr + ck, nsplit, split_stride));
             const float b = scale(split_fin1(pb, pr + ck + half, nsplit, split_stride));
             Kpool[base + i] = (KVT)(a * c - b * sn);
@@ -539,19 +586,34 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qout, 
     }
 }
 
+template <typename KVT>
+static void launch_rope_kv_t(dim3 grid, hipStream_t s, float* qout, void* Kpool, void* Vpool, const float* part,
+                             int nsplit, int64_t split_stride, int qkv_ld, const int32_t* tok2seq,
+                             const int32_t* tok_pos, const int64_t* kv_base, int n_heads, int n_kv_heads, int hd,
+                             int64_t head_stride, const float* cs, const RowNorm& rn) {
+    // one split (large prompt steps): one load per partial, not eight clamped ones
+    if (nsplit <= 1)
+        hipLaunchKernelGGL((rope_kv_kernel<KVT, 1>), grid, dim3(256), 0, s, qout, (KVT*)Kpool, (KVT*)Vpool, part,
+                           nsplit, split_stride, qkv_ld, tok2seq, tok_pos, kv_base, n_heads, n_kv_heads, hd,
+                           head_stride, cs, rn);
+    else
+        hipLaunchKernelGGL((rope_kv_kernel<KVT, 8>), grid, dim3(256), 0, s, qout, (KVT*)Kpool, (KVT*)Vpool, part,
+                           nsplit, split_stride, qkv_ld, tok2seq, tok_pos, kv_base, n_heads, n_kv_heads, hd,
+                           head_stride, cs, rn);
+}
+
 int launch_rope_kv(float* qout, void* Kpool, void* Vpool, const float* part, int nsplit, int64_t split_stride,
                    int qkv_ld, const int32_t* tok2seq, const int32_t* tok_pos, const int64_t* kv_base, int T,
                    int n_heads, int n_kv_heads, int hd, int64_t head_stride, const float* cs, const RowNorm& rn,
                    bool kv_f16, hipStream_t s) {
     if (T <= 0) return 0;
+    const dim3 grid((n_heads + n_kv_heads + 3) / 4, T);
     if (kv_f16)
-        hipLaunchKernelGGL(rope_kv_kernel<_Float16>, dim3((n_heads + n_kv_heads + 3) / 4, T), dim3(256), 0, s, qout,
-                           (_Float16*)Kpool, (_Float16*)Vpool, part, nsplit, split_stride, qkv_ld, tok2seq, tok_pos,
-                           kv_base, n_heads, n_kv_heads, hd, head_stride, cs, rn);
+        launch_rope_kv_t<_Float16>(grid, s, qout, Kpool, Vpool, part, nsplit, split_stride, qkv_ld, tok2seq, tok_pos,
+                                   kv_base, n_heads, n_kv_heads, hd, head_stride, cs, rn);
     else
-        hipLaunchKernelGGL(rope_kv_kernel<float>, dim3((n_heads + n_kv_heads + 3) / 4, T), dim3(256), 0, s, qout,
-                           (float*)Kpool, (float*)Vpool, part, nsplit, split_stride, qkv_ld, tok2seq, tok_pos,
-                           kv_base, n_heads, n_kv_heads, hd, head_stride, cs, rn);
+        launch_rope_kv_t<float>(grid, s, qout, Kpool, Vpool, part, nsplit, split_stride, qkv_ld, tok2seq, tok_pos,
+                                kv_base, n_heads, n_kv_heads, hd, head_stride, cs, rn);
     SH_CHECK_LAUNCH();
     return 0;
 }

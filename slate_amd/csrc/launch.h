@@ -18,7 +18,10 @@ int launch_rope_rows(float* x, const int32_t* pos, int n_rows, int n_heads, int 
 // Fused engine epilogues; `a` (nullable) receives the Q4_K activation operand
 // of rows_pad rows (rows past `rows` zero), y (nullable) the f32 rows.
 int launch_rmsnorm_act(float* y, float* x, const float* delta, int nsplit, int64_t split_stride, const float* w,
-                       int rows, int D, float eps, const Act16* a, hipStream_t s);
+                       int rows, int D, float eps, const Act16* a, hipStream_t s, const int32_t* pick = nullptr,
+                       int src_rows = 0);
+// inv[r] = the RMSNorm factor of row r < rows (RowNorm::inv of the consumers).
+int launch_row_inv(float* inv, const RowNorm& rn, int rows, hipStream_t s);
 int launch_silu_act(float* y, const float* gate, const float* up, int rows, int H, int nsplit,
                     int64_t split_stride, int64_t ld, const Act16* a, const RowNorm& rn, hipStream_t s);
 // K/V rows are written as f32, or rounded to f16 when kv_f16.

@@ -40,7 +40,8 @@ __device__ __forceinline__ float split_sum1(const float* p, int n, int64_t strid
 // order and with the same result as split_sum4 / split_sum1.
 template <int N = 8> struct Split4N { float4 t[N]; };
 using Split4 = Split4N<8>;
-struct Split1 { float t[8]; };
+template <int N = 8> struct Split1N { float t[N]; };
+using Split1 = Split1N<8>;
 template <int N = 8>
 __device__ __forceinline__ Split4N<N> split_load4(const float* p, int n, int64_t stride) {
     Split4N<N> r;
@@ -48,10 +49,11 @@ __device__ __forceinline__ Split4N<N> split_load4(const float* p, int n, int64_t
     for (int i = 0; i < N; ++i) r.t[i] = *(const float4*)(p + (int64_t)min(i, max(n - 1, 0)) * stride);
     return r;
 }
-__device__ __forceinline__ Split1 split_load1(const float* p, int n, int64_t stride) {
-    Split1 r;
+template <int N = 8>
+__device__ __forceinline__ Split1N<N> split_load1(const float* p, int n, int64_t stride) {
+    Split1N<N> r;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) r.t[i] = p[(int64_t)min(i, max(n - 1, 0)) * stride];
+    for (int i = 0; i < N; ++i) r.t[i] = p[(int64_t)min(i, max(n - 1, 0)) * stride];
     return r;
 }
 // (N = 16 loads sixteen partials up front: one round trip up to 16 splits)
@@ -71,12 +73,13 @@ __device__ __forceinline__ float4 split_fin4(const Split4N<N>& r, const float* p
     }
     return s;
 }
-__device__ __forceinline__ float split_fin1(const Split1& r, const float* p, int n, int64_t stride) {
+template <int N = 8>
+__device__ __forceinline__ float split_fin1(const Split1N<N>& r, const float* p, int n, int64_t stride) {
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < N; ++i)
         if (i < n) s += r.t[i];
-    for (int k = 8; k < n; k += 8) {
+    for (int k = N; k < n; k += 8) {
         float t[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) t[i] = p[(int64_t)min(k + i, n - 1) * stride];

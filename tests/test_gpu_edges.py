@@ -4,8 +4,12 @@ each compared with float64 under a bound that follows from its arithmetic.
 import numpy as np
 import pytest
 
+import slate_amd
+from oracle.pyoracle import OracleModel
 from slate_amd import DeviceBuffer as DB
 from slate_amd import check
+from slate_amd.synth import make_llama
+from tests.helpers import Q4, Q4_SEED, relerr
 
 pytestmark = pytest.mark.gpu
 
@@ -213,3 +217,27 @@ def test_q4k_matvec_activation_paths(hip, M, K):
     # up to three passes, 4 + 32 sums: under 80 roundings of the absolute sum
     x6 = x.astype(np.float64)
     assert np.all(np.abs(got[:M] - w @ x6) <= 80 * EPS * (size @ np.abs(x6)))
+
+
+@pytest.mark.parametrize("lens", [(100, 27), (101, 27), (64, 65), (1, 120, 3, 90)])
+def test_prompt_steps_around_the_shared_row_factor(orc, lens):
+    """Prompt steps of 127 rows (each consumer sums a row's squares itself), 128
+    and more (one kernel does), the last rows alone normalised for the LM
+    head; then a decode step.  Against the oracle token by token; 1e-4 is the
+    bound between any two orders of the engine's sums in this suite."""
+    t = make_llama(Q4, Q4_SEED, quant="q4k")
+    m = slate_amd.Llama.from_tensors(Q4, t, max_slots=len(lens), max_tokens=sum(lens))
+    om = OracleModel(orc, Q4, t)
+    rng = np.random.default_rng(sum(lens))
+    prompts = [rng.integers(0, Q4.vocab, n).astype(np.int32) for n in lens]
+    ss = [m.session() for _ in lens]
+    rc, lg, _ = m.step(ss, lens, np.concatenate(prompts))
+    check(rc, "prompt step")
+    rc, lg2, _ = m.step(ss, [1] * len(lens), np.full(len(lens), 5, np.int32))
+    check(rc, "decode step")
+    for i, p in enumerate(prompts):
+        o = om.session()
+        _, want = o.prefill(p)
+        assert relerr(lg[i], want) < 1e-4, i
+        _, want = o.decode(5)
+        assert relerr(lg2[i], want) < 1e-4, i
