@@ -1240,6 +1240,12 @@ int launch_attention_blocks(float* out, const float* q, const void* Kp, const vo
             rc = launch_attention_prompt(q, (const float*)Kp, (const float*)Vp, tok2seq, tok_pos, kv_base, pre_t0,
                                          pre_n, n_pre, Hq, Hkv, HD, head_stride, nch_max, po, pml, s, a.ev0);
             if (rc) return rc;
+        } else if (!prefill && !pairs_ready && !kv_f16 && wave_kernel() && n_dec > ATT_WAVE_MAX_TOKENS &&
+                   // past the decode batches prompt chunks are among the
+                   // tokens (65 to 71 tokens with two to four chunks: 1.1 to 1.7x)
+                   (HD == 32 || HD == 64 || HD == 128)) {
+            rc = launch_attention_runs(q, (const float*)Kp, (const float*)Vp, tok2seq, tok_pos, kv_base, dec_t0,
+                                       n_dec, Hq, Hkv, HD, head_stride, nch_max, po, pml, pairs, s, a.ev0);
         } else if (!prefill && (HD == 32 || HD == 64 || HD == 128)) {
             if (!pairs_ready) {
                 SH_LAUNCH(a.ev0, nullptr, attn_pairs_kernel, dim3(1), dim3(1024), 0, s, dec_t0, n_dec, tok_pos,

@@ -241,3 +241,81 @@ def test_prompt_steps_around_the_shared_row_factor(orc, lens):
         assert relerr(lg[i], want) < 1e-4, i
         _, want = o.decode(5)
         assert relerr(lg2[i], want) < 1e-4, i
+
+
+def _ragged_case(rng, order):
+    """(sequence, position) per token: runs of several lengths around the
+    units of 16 / G tokens and the chunks of 256 keys, joined, broken, or in
+    an order in which hardly any token follows another."""
+    runs = [(0, 0, 33), (1, 250, 9), (2, 0, 1), (2, 1, 4), (3, 511, 2), (4, 700, 17), (0, 33, 2), (5, 3, 1)]
+    tok = [(s, p0 + i) for s, p0, n in runs for i in range(n)]
+    tok += [(6, 40), (6, 40), (6, 39), (6, 38)]             # repeated and falling positions
+    if order == "shuffled":
+        tok = [tok[i] for i in rng.permutation(len(tok))]
+    elif order == "reversed":
+        tok = tok[::-1]
+    elif order == "long":                                   # runs over the list kernel's 1024 entries
+        tok = tok + [(7, i) for i in range(720)] + [(4, i) for i in range(250)] + [(1, 5)]
+    return tok
+
+
+@pytest.mark.parametrize("hd,Hq,Hkv,order", [(128, 8, 2, "joined"), (128, 2, 2, "joined"), (128, 8, 1, "shuffled"),
+                                             (64, 4, 2, "joined"), (64, 8, 2, "reversed"), (32, 8, 8, "joined"),
+                                             (32, 16, 2, "long"), (32, 3, 3, "long"), (64, 24, 3, "joined")])
+def test_attention_runs(hip, hd, Hq, Hkv, order):
+    """More than 64 query tokens: runs share their K/V rows, whatever order
+    the tokens come in.  Every cache row that no token may see is NaN."""
+    rng = np.random.default_rng(hd * Hq + len(order))
+    S, nslot = 768, 8
+    tok = _ragged_case(rng, order)
+    T = len(tok)
+    seq = np.array([s for s, _ in tok], np.int32)
+    pos = np.array([p for _, p in tok], np.int32)
+    last = [max([p for s, p in tok if s == b], default=-1) for b in range(nslot)]
+    K = rng.normal(0, 1, (nslot, Hkv, S, hd)).astype(np.float32)
+    V = rng.normal(0, 1, (nslot, Hkv, S, hd)).astype(np.float32)
+    for b in range(nslot):
+        K[b, :, last[b] + 1:] = np.nan
+        V[b, :, last[b] + 1:] = np.nan
+    base = np.arange(nslot, dtype=np.int64)[::-1] * (Hkv * S * hd)
+    q = rng.normal(0, 1, (T, Hq, hd)).astype(np.float32)
+
+    def call(Kc, Vc):
+        out = DB((T * Hq * hd + 64) * 4)
+        out.upload(np.full(T * Hq * hd + 64, 7.0, np.float32))
+        check(hip.lib.slate_hip_attention_ragged(
+            out.p, DB.from_array(q).p, DB.from_array(Kc[::-1].copy()).p, DB.from_array(Vc[::-1].copy()).p,
+            DB.from_array(seq).p, DB.from_array(pos).p, DB.from_array(base.copy()).p, T, Hq, Hkv, hd, S * hd, S),
+            "attention_ragged")
+        got = host(out, (T * Hq * hd + 64,))
+        assert np.all(got[T * Hq * hd:] == 7.0)
+        return got[:T * Hq * hd].reshape(T, Hq, hd)
+
+    got = call(K, V)
+    G = Hq // Hkv
+    q6, K6, V6 = q.astype(np.float64), K.astype(np.float64), V.astype(np.float64)
+    for t in range(T):
+        L = pos[t] + 1
+        k, v = K6[seq[t], :, :L].repeat(G, 0), V6[seq[t], :, :L].repeat(G, 0)
+        s = np.einsum("hd,hld->hl", q6[t], k) / np.sqrt(hd)
+        mag = np.einsum("hd,hld->hl", np.abs(q6[t]), np.abs(k)).max() / np.sqrt(hd)
+        p = np.exp(s - s.max(-1, keepdims=True))
+        p /= p.sum(-1, keepdims=True)
+        # a score is hd products and sums; its error moves a weight by that
+        # much twice (numerator and sum); then at most 256 + 64 roundings
+        bound = (2 * (hd + 8) * EPS * mag + (min(L, 256) + 64) * EPS) * np.einsum("hl,hld->hd", p, np.abs(v))
+        assert np.all(np.abs(got[t] - np.einsum("hl,hld->hd", p, v)) <= bound), (t, tok[t])
+
+    # an infinite V row reaches the tokens that see it and no others, with
+    # every other token's bits as they were but for the order of its sums
+    V[1, :, 255] = np.inf
+    V[0, :, 17, 3] = np.nan
+    again = call(K, V)
+    for t in range(T):
+        if seq[t] == 1 and pos[t] >= 255:
+            assert not np.any(np.isfinite(again[t])), (t, tok[t])
+        elif seq[t] == 0 and pos[t] >= 17:
+            assert np.all(np.isnan(again[t][:, 3])) and np.all(np.isfinite(np.delete(again[t], 3, -1)))
+        else:
+            # (the last tokens of a run take the exact path of their unit)
+            assert np.allclose(again[t], got[t], rtol=0, atol=64 * EPS * 8), (t, tok[t])
