@@ -9,7 +9,7 @@
 // each unit's K and V rows once for all its rows.  A token that follows no
 // other is a unit of its own.
 //
-// A unit's four waves own 64 keys each.  Scores are S^T = K Q^T (16 keys x 16
+// A unit's four waves own up to 64 keys each.  Scores are S^T = K Q^T (16 keys x 16
 // rows per MFMA tile, 4 dims a step): a lane holds scores of one row, keys
 // 4g .. 4g+3 of each tile, which is the layout that O^T += V^T P^T takes as
 // its second operand, so probabilities never leave their registers.  A wave
@@ -23,11 +23,13 @@
 //
 // Bound: the f32 MFMA (64 flops a clock and SIMD; busy 40 % of the time) and
 // the vector ALUs beside it (softmax, tree sums).  13 decode tokens at ~900
-// keys and three chunks of 121-172 tokens (32 q / 8 kv heads of 128): 132 us
-// token by token, 88 here; with the chunks alone in a call 1.3 to 1.9 times
-// as fast from hd 64 x 16 heads to hd 128 x 64.  32 rows a unit halve the K/V
-// traffic but leave two waves a SIMD: 97 us.  Chains of four MFMAs take 128
-// registers and 80 us, but round 3 to 10 % worse.
+// keys and three chunks of 121-172 tokens (32 q / 8 kv heads of 128), the
+// whole call: 139 us token by token, 89 here; 32 q and kv heads of 128, four
+// chunks of up to 98 tokens: 55 and 28 us; 16 q / 4 kv heads of 64, four of up
+// to 68 beside nine decode tokens: 32 and 23.  Lone tokens gain nothing (128
+// at ~300 keys 92 and 90 us, 300 at ~60 keys 23 and 25).  32 rows a unit halve the K/V
+// traffic but leave two waves a SIMD: 102 us.  Chains of four MFMAs fit 128
+// registers (four waves; 86 us where these took 93), but round 3 to 10 % worse.
 #include <algorithm>
 #include <cfloat>
 
@@ -38,7 +40,7 @@
 namespace slate_hip {
 
 constexpr int ARN_CHUNK = 256;       // keys per unit: the merge kernel's chunk
-constexpr int ARN_KW = 64;           // keys per wave
+constexpr int ARN_KW = 64;           // keys per wave, at most
 constexpr int ARN_ROWS = 16;         // query rows per unit
 constexpr int ARN_LIST = 1024;       // threads of the list kernel
 
@@ -159,8 +161,11 @@ __device__ __forceinline__ void attn_run_unit(const float* q, const float* Kp, c
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int k0 = un.c * ARN_CHUNK;
     const int nk = min(un.p0 + un.n - k0, ARN_CHUNK);       // keys some row of the unit sees
-    const int kw0 = wv * ARN_KW;
-    const bool active = kw0 < nk;
+    // the chunk's keys in whole tiles over the four waves (a chunk of 130 keys
+    // as 48 + 48 + 34, not 64 + 64 + 2)
+    const int kw = (nk + 63) / 64 * 16, kw0 = wv * kw;
+    const int kn = min(nk - kw0, kw);                       // the wave's keys
+    const bool active = kn > 0;
     const float scale = 1.0f / sqrtf((float)HD);
     const float* Kh = Kp + un.kv;
     const float* Vh = Vp + un.kv;
@@ -221,37 +226,36 @@ __device__ __forceinline__ void attn_run_unit(const float* q, const float* Kp, c
         // bits where these show 1.2e-7)
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
+            s[kt] = floatx4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+            if (16 * kt >= kn) continue;
             wait_copies();
             floatx4 kf[NT];
 #pragma unroll
             for (int m = 0; m < NT; ++m) kf[m] = *(const floatx4*)(so + Geo::at(j, 16 * m + 4 * g));
             wait_lds();                                     // the tile is in registers: the next one may land
-            if (kt + 1 < KT) copy(Kh, kt + 1);
+            if (16 * (kt + 1) < kn) copy(Kh, kt + 1);
             else copy(Vh, 0);
             __builtin_amdgcn_sched_barrier(0);
-            s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
-            if (kw0 + 16 * kt < nk) {
-                floatx4 tr[4];                              // pending partial sums of the pairwise tree
+            floatx4 tr[4];                                  // pending partial sums of the pairwise tree
 #pragma unroll
-                for (int m = 0; m < NT; ++m) {
-                    floatx4 t[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+            for (int m = 0; m < NT; ++m) {
+                floatx4 t[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-                    for (int e = 0; e < 2; ++e)
+                for (int e = 0; e < 2; ++e)
 #pragma unroll
-                        for (int x = 0; x < 2; ++x)
-                            t[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[m][2 * x + e], qf[m][2 * x + e], t[x],
-                                                                        0, 0, 0);
-                    t[0] += t[1];
-                    int lv = 0;
+                    for (int x = 0; x < 2; ++x)
+                        t[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[m][2 * x + e], qf[m][2 * x + e], t[x],
+                                                                    0, 0, 0);
+                t[0] += t[1];
+                int lv = 0;
 #pragma unroll
-                    for (; (m >> lv) & 1; ++lv) t[0] = tr[lv] + t[0];
-                    tr[lv] = t[0];
-                    // two chains at a time: left to itself the scheduler starts
-                    // more than the registers hold
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                s[kt] = tr[NT == 8 ? 3 : (NT == 4 ? 2 : 1)];
+                for (; (m >> lv) & 1; ++lv) t[0] = tr[lv] + t[0];
+                tr[lv] = t[0];
+                // two chains at a time: left to itself the scheduler starts
+                // more than the registers hold
+                __builtin_amdgcn_sched_barrier(0);
             }
+            s[kt] = tr[NT == 8 ? 3 : (NT == 4 ? 2 : 1)];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int k = kw0 + 16 * kt + 4 * g + i;
@@ -299,6 +303,7 @@ __device__ __forceinline__ void attn_run_unit(const float* q, const float* Kp, c
         bool bad = false;
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
+            if (16 * kt >= kn) continue;
             wait_copies();
             // lane (j, g): key 4g + i, dims VW*j .. of each VW*16-dim block
             vf_t vf[4][NB];
@@ -307,31 +312,29 @@ __device__ __forceinline__ void attn_run_unit(const float* q, const float* Kp, c
 #pragma unroll
                 for (int b = 0; b < NB; ++b) vf[i][b] = *(const vf_t*)(so + Geo::at(4 * g + i, 16 * VW * b + VW * j));
             wait_lds();
-            if (kt + 1 < KT) copy(Vh, kt + 1);
+            if (16 * (kt + 1) < kn) copy(Vh, kt + 1);
             __builtin_amdgcn_sched_barrier(0);
-            if (kw0 + 16 * kt < nk) {
-                if (kw0 + 16 * kt + 15 > diag)
+            if (kw0 + 16 * kt + 15 > diag)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < 4; ++i)
 #pragma unroll
-                        for (int b = 0; b < NB; ++b)
+                    for (int b = 0; b < NB; ++b)
 #pragma unroll
-                            for (int c = 0; c < VW; ++c) bad |= !(fabsf(vf[i][b][c]) <= FLT_MAX);
+                        for (int c = 0; c < VW; ++c) bad |= !(fabsf(vf[i][b][c]) <= FLT_MAX);
 #pragma unroll
-                for (int b = 0; b < NB; ++b)
+            for (int b = 0; b < NB; ++b)
 #pragma unroll
-                    for (int c = 0; c < VW; ++c) {
-                        floatx4 t[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+                for (int c = 0; c < VW; ++c) {
+                    floatx4 t[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-                        for (int i = 0; i < 2; ++i)
+                    for (int i = 0; i < 2; ++i)
 #pragma unroll
-                            for (int x = 0; x < 2; ++x)
-                                t[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[2 * x + i][b][c], s[kt][2 * x + i],
-                                                                            t[x], 0, 0, 0);
-                        acc[b * VW + c] += t[0] + t[1];
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-            }
+                        for (int x = 0; x < 2; ++x)
+                            t[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[2 * x + i][b][c], s[kt][2 * x + i],
+                                                                        t[x], 0, 0, 0);
+                    acc[b * VW + c] += t[0] + t[1];
+                    __builtin_amdgcn_sched_barrier(0);
+                }
         }
         if (__any(bad)) {
             // some V value there is not finite: each row over its own keys alone
@@ -342,7 +345,7 @@ __device__ __forceinline__ void attn_run_unit(const float* q, const float* Kp, c
 #pragma unroll
             for (int n = 0; n < NT; ++n) acc[n] = floatx4{0.f, 0.f, 0.f, 0.f};
             wait_lds();
-            for (int k = 0; k < ARN_KW && kw0 + k < nk; ++k)
+            for (int k = 0; k < kn; ++k)
                 if (k0 + kw0 + k <= un.p0 + min(j / G, un.n - 1)) {
                     const float pk = so[j * ARN_KW + k];
                     const float* vr = Vh + (int64_t)(kw0 + k) * HD;
@@ -369,7 +372,7 @@ __device__ __forceinline__ void attn_run_unit(const float* q, const float* Kp, c
         if (g == 0) s_l[wv * R + j] = sum;
     }
     __syncthreads();
-    const int nw = (nk + ARN_KW - 1) / ARN_KW;              // waves that had keys
+    const int nw = (nk + kw - 1) / kw;                      // waves that had keys
     for (int idx = tid; idx < R * CPR; idx += 256) {
         const int r = idx / CPR, d = 4 * (idx % CPR), i = r / G;
         if (i >= un.n || un.p0 + i < k0) continue;          // the merge reads no chunk past a token's end
