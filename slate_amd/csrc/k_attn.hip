@@ -1166,6 +1166,12 @@ static bool wave_kernel() { return knobs().attn_wave != 0; }
 // HBM); prompt tokens, whose K/V re-reads hit L2, run the phased kernel at
 // its higher occupancy.
 constexpr int ATT_WAVE_MAX_TOKENS = 64;
+// Past the decode batches prompt chunks are among the tokens, and runs of
+// them share their K/V rows (65 to 71 tokens with two to four chunks: 1.1 to
+// 1.7x; k_attn_run.hip).
+static bool runs_kernel(int HD, int n_dec, bool kv_f16) {
+    return wave_kernel() && n_dec > ATT_WAVE_MAX_TOKENS && !kv_f16 && (HD == 32 || HD == 64 || HD == 128);
+}
 
 template <int HD, int G, typename KVT>
 static void launch_dec_t(dim3 grid, hipStream_t s, const AttnArgs& a) {
@@ -1240,10 +1246,8 @@ int launch_attention_blocks(float* out, const float* q, const void* Kp, const vo
             rc = launch_attention_prompt(q, (const float*)Kp, (const float*)Vp, tok2seq, tok_pos, kv_base, pre_t0,
                                          pre_n, n_pre, Hq, Hkv, HD, head_stride, nch_max, po, pml, s, a.ev0);
             if (rc) return rc;
-        } else if (!prefill && !pairs_ready && !kv_f16 && wave_kernel() && n_dec > ATT_WAVE_MAX_TOKENS &&
-                   // past the decode batches prompt chunks are among the
-                   // tokens (65 to 71 tokens with two to four chunks: 1.1 to 1.7x)
-                   (HD == 32 || HD == 64 || HD == 128)) {
+        } else if (runs_kernel(HD, n_dec, kv_f16) && !prefill && !pairs_ready && head_stride % 4 == 0 &&
+                   (((uintptr_t)q | (uintptr_t)Kp | (uintptr_t)Vp) & 15) == 0) {
             rc = launch_attention_runs(q, (const float*)Kp, (const float*)Vp, tok2seq, tok_pos, kv_base, dec_t0,
                                        n_dec, Hq, Hkv, HD, head_stride, nch_max, po, pml, pairs, s, a.ev0);
         } else if (!prefill && (HD == 32 || HD == 64 || HD == 128)) {
