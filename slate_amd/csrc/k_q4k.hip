@@ -224,7 +224,11 @@ __device__ __forceinline__ half8_t q4k_bop(const WTile& w, const WScale& c, int 
 // block into registers before computing the current one, and after it
 // writes them into the other LDS buffer in the operand layout (act16.h), the
 // same values the operand kernel would write.
-template <int R, bool TILED, int WAVES = 4, int NT = 1, bool CONV = false>
+//
+// DIRECT (an unsplit plan of one tensor): the rows below tg.row_end go to the
+// caller's output.  An instantiation of its own: a test at every store of
+// the partials makes each a branch, for rows that the engine always pads.
+template <int R, bool TILED, int WAVES = 4, int NT = 1, bool CONV = false, bool DIRECT = false>
 __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, const uint4* frag,
                                                              float* __restrict__ out, int64_t ldo,
                                                              int64_t split_stride, int nblk, int bps, int early,
@@ -429,7 +433,6 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, cons
         if (b < nb) step(w1, w0, b);
     }
     if (!active) return;
-    const bool all = tg.row_end >= 16 * NT;           // wave-uniform: partials have every padded row
     float* o = out + (int64_t)blockIdx.y * split_stride + col;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -438,9 +441,10 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, cons
 #pragma unroll
             for (int n = 0; n < NT; ++n)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (all || 16 * n + 4 * g + i < tg.row_end)
-                        o[(int64_t)(16 * n + 4 * g + i) * ldo + row] = acc[r][n][i];
+                for (int i = 0; i < 4; ++i) {
+                    const int b = 16 * n + 4 * g + i;
+                    if (!DIRECT || b < tg.row_end) o[(int64_t)b * ldo + row] = acc[r][n][i];
+                }
         }
     }
 }
@@ -848,24 +852,31 @@ static void dec_plan(const int* tiles, int n, int nblk, int s_max, int bps_max, 
     *S_out = S_out_v;
 }
 
-template <int R, bool TILED>
-static void launch_dec(const Q4kTargets& tg, const Act16& a, float* out, int64_t ldo, int64_t ss, int nblk,
-                       int bps, int nsplit, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+template <int R, bool TILED, int NT, bool DIRECT>
+static void launch_dec_nt(const Q4kTargets& tg, const Act16& a, float* out, int64_t ldo, int64_t ss, int nblk,
+                          int bps, int nsplit, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
     const int W = dec_waves();
     const int early = knobs().q4k_early;
     const dim3 grid((tg.grp_end + W - 1) / W, nsplit);
     const uint4* fr = (const uint4*)a.frag;
+    if (W == 8)
+        SH_LAUNCH(e0, e1, (q4k_dec_kernel<R, TILED, 8, NT, false, DIRECT>), grid, dim3(512), 0, s, tg, fr, out, ldo,
+                  ss, nblk, bps, early, (const float*)nullptr, (int64_t)0, 0);
+    else
+        SH_LAUNCH(e0, e1, (q4k_dec_kernel<R, TILED, 4, NT, false, DIRECT>), grid, dim3(256), 0, s, tg, fr, out, ldo,
+                  ss, nblk, bps, early, (const float*)nullptr, (int64_t)0, 0);
+}
+
+template <int R, bool TILED>
+static void launch_dec(bool direct, const Q4kTargets& tg, const Act16& a, float* out, int64_t ldo, int64_t ss,
+                       int nblk, int bps, int nsplit, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
     if (a.rows_pad == 32) {
-        if (W == 8) SH_LAUNCH(e0, e1, (q4k_dec_kernel<R, TILED, 8, 2>), grid, dim3(512), 0, s, tg, fr, out, ldo, ss, nblk, bps,
-                  early, (const float*)nullptr, (int64_t)0, 0);
-        else SH_LAUNCH(e0, e1, (q4k_dec_kernel<R, TILED, 4, 2>), grid, dim3(256), 0, s, tg, fr, out, ldo, ss, nblk, bps,
-                  early, (const float*)nullptr, (int64_t)0, 0);
-        return;
+        if (direct) launch_dec_nt<R, TILED, 2, true>(tg, a, out, ldo, ss, nblk, bps, nsplit, s, e0, e1);
+        else launch_dec_nt<R, TILED, 2, false>(tg, a, out, ldo, ss, nblk, bps, nsplit, s, e0, e1);
+    } else {
+        if (direct) launch_dec_nt<R, TILED, 1, true>(tg, a, out, ldo, ss, nblk, bps, nsplit, s, e0, e1);
+        else launch_dec_nt<R, TILED, 1, false>(tg, a, out, ldo, ss, nblk, bps, nsplit, s, e0, e1);
     }
-    if (W == 8) SH_LAUNCH(e0, e1, (q4k_dec_kernel<R, TILED, 8, 1>), grid, dim3(512), 0, s, tg, fr, out, ldo, ss, nblk, bps,
-                  early, (const float*)nullptr, (int64_t)0, 0);
-    else SH_LAUNCH(e0, e1, (q4k_dec_kernel<R, TILED, 4, 1>), grid, dim3(256), 0, s, tg, fr, out, ldo, ss, nblk, bps,
-                  early, (const float*)nullptr, (int64_t)0, 0);
 }
 
 constexpr int PF_R = 2, PF_WAVES = 8;
@@ -1017,14 +1028,15 @@ int launch_q4k(const Q4kTarget* t, int n, bool tiled, const Act16& a, float* out
     tg.n = n;
     tg.grp_end = grp;
     target(tg, S);
+    const bool dir = direct && S == 1;
     if (tiled) {
-        if (R == 4) launch_dec<4, true>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
-        else if (R == 2) launch_dec<2, true>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
-        else launch_dec<1, true>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
+        if (R == 4) launch_dec<4, true>(dir, tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
+        else if (R == 2) launch_dec<2, true>(dir, tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
+        else launch_dec<1, true>(dir, tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
     } else {
-        if (R == 4) launch_dec<4, false>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
-        else if (R == 2) launch_dec<2, false>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
-        else launch_dec<1, false>(tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
+        if (R == 4) launch_dec<4, false>(dir, tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
+        else if (R == 2) launch_dec<2, false>(dir, tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
+        else launch_dec<1, false>(dir, tg, a, out, ldo, split_stride, nblk, bps, S, s, ev_start, ev_stop);
     }
     SH_CHECK_LAUNCH();
     *S_out = S;
@@ -1074,7 +1086,6 @@ int launch_q4k_conv(const Q4kTarget& t, bool tiled, const float* X, int64_t ldx,
     tg.grp0[0] = 0;
     tg.n = 1;
     tg.grp_end = (tiles + R - 1) / R;
-    tg.row_end = 16;
     if (tiled) {
         if (R == 4) launch_dec_conv<4, true>(tg, X, ldx, rows, out, ldo, split_stride, nblk, bps, S, s);
         else if (R == 2) launch_dec_conv<2, true>(tg, X, ldx, rows, out, ldo, split_stride, nblk, bps, S, s);
