@@ -126,12 +126,12 @@ int launch_sum_splits(float* Y, const float* part, int nsplit, int rows, int row
                       hipStream_t s);
 
 // Per-row RMSNorm factor deferred to the consumer of a matmul: ssq holds
-// the sums of squares per 256-element block [rows][D/256] (nullptr = none).
+// the sums of squares per 256-element block [rows][D/256] (nullptr = none),
+// or with nblk = 0 the rows' factors, computed once (prompt steps).
 struct RowNorm {
     const float* ssq;
     int nblk, D;
     float eps;
-    const float* inv = nullptr;     // the rows' factors, where a kernel computed them once (prompt steps)
 };
 
 // Up to three Q4_K tensors sharing one input, fused into one launch; tensor i

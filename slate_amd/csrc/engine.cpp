@@ -453,7 +453,7 @@ constexpr int ROW_INV_ROWS = 128;
 int norm_factors(slate_hip_llama* m, RowNorm& rn, int T, hipStream_t s) {
     if (!rn.ssq || T < ROW_INV_ROWS || m->step_one_each) return 0;
     const int rc = launch_row_inv(m->inv, rn, T, s);
-    if (rc == 0) rn.inv = m->inv;
+    if (rc == 0) rn.ssq = m->inv, rn.nblk = 0;
     return rc;
 }
 

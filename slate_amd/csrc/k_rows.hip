@@ -427,7 +427,7 @@ __device__ __forceinline__ void silu_act_body(float* __restrict__ y, const float
         const Split4N<NPRE> pu = split_load4<NPRE>(upp, nsplit, split_stride);
         RmsPre rp;
         float inv = 0.f;
-        if constexpr (INV) inv = rn.inv[r];
+        if constexpr (INV) inv = rn.ssq[r];
         else if (rn.ssq) rp = row_rms_load(rn.ssq, r, rn.nblk);
         float4 g = split_fin4(pg, gp, nsplit, split_stride), u = split_fin4(pu, upp, nsplit, split_stride);
         if (rn.ssq) {   // gate and up are linear in the normalised row
@@ -474,22 +474,23 @@ int launch_silu_act(float* y, const float* gate, const float* up, int rows, int 
     // written by 8-row half tiles
     const Act16 ao = a ? *a : Act16{};
     const int act = a ? 1 : 0;
+    const bool factors = rn.ssq && !rn.nblk;
     if (nsplit <= 1 && a && a->rows_pad > 16) {
         const dim3 tg(nblk, a->rows_pad / 8);
-        if (rn.inv)
+        if (factors)
             hipLaunchKernelGGL(silu_act_tile_kernel<true>, tg, dim3(512), 0, s, y, gate, up, rows, H, nsplit,
                                split_stride, ld, ao, rn);
         else
             hipLaunchKernelGGL(silu_act_tile_kernel<false>, tg, dim3(512), 0, s, y, gate, up, rows, H, nsplit,
                                split_stride, ld, ao, rn);
     } else if (nsplit <= 1) {
-        if (rn.inv)
+        if (factors)
             hipLaunchKernelGGL((silu_act_kernel<1, true>), grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit,
                                split_stride, ld, ao, act, rn);
         else
             hipLaunchKernelGGL((silu_act_kernel<1, false>), grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit,
                                split_stride, ld, ao, act, rn);
-    } else if (rn.inv) {
+    } else if (factors) {
         hipLaunchKernelGGL((silu_act_kernel<8, true>), grid, dim3(64), 0, s, y, gate, up, rows, H, nsplit,
                            split_stride, ld, ao, act, rn);
     } else {
@@ -547,8 +548,11 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qout, 
     // the position-dependent ones (rotation table, KV row).
     RmsPre rp;
     float inv = 1.0f;
-    if (rn.inv) inv = rn.inv[t];
-    else if (rn.ssq) rp = row_rms_load(rn.ssq, t, rn.nblk);
+    const bool sums = rn.nblk > 0;                 // else the factor itself
+    if (rn.ssq) {
+        if (sums) rp = row_rms_load(rn.ssq, t, rn.nblk);
+        else inv = rn.ssq[t];
+    }
     auto scale = [&](float v) { return rn.ssq ? v * inv : v; };
     if (u < n_heads) {
         for (int i = lane; i < half; i += 64) {
@@ -557,7 +561,7 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qout, 
             const Split1N<NPRE> pb = split_load1<NPRE>(pr + c0 + half, nsplit, split_stride);
             const float c = cs[((size_t)ap * half + i) * 2 + 0];
             const float sn = sg * cs[((size_t)ap * half + i) * 2 + 1];
-            if (rn.ssq && !rn.inv) inv = row_rms_fin(rp, rn.ssq, t, rn.nblk, rn.D, rn.eps);
+            if (rn.ssq && sums) inv = row_rms_fin(rp, rn.ssq, t, rn.nblk, rn.D, rn.eps);
             const float a = scale(split_fin1(pa, pr + c0, nsplit, split_stride));
             const float b = scale(split_fin1(pb, pr + c0 + half, nsplit, split_stride));
             qout[(size_t)t * D + c0] = a * c - b * sn;
@@ -575,7 +579,7 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(float* __restrict__ qout, 
             const float c = cs[((size_t)ap * half + i) * 2 + 0];
             const float sn = sg * cs[((size_t)ap * half + i) * 2 + 1];
             const int64_t base = kv_base[seq] + (int64_t)kh * head_stride + (int64_t)p * hd;
-            if (rn.ssq && !rn.inv) inv = row_rms_fin(rp, rn.ssq, t, rn.nblk, rn.D, rn.eps);
+            if (rn.ssq && sums) inv = row_rms_fin(rp, rn.ssq, t, rn.nblk, rn.D, rn.eps);
             const float a = scale(split_fin1(pa, pr + ck, nsplit, split_stride));
             const float b = scale(split_fin1(pb, pr + ck + half, nsplit, split_stride));
             Kpool[base + i] = (KVT)(a * c - b * sn);

@@ -20,7 +20,7 @@ int launch_rope_rows(float* x, const int32_t* pos, int n_rows, int n_heads, int 
 int launch_rmsnorm_act(float* y, float* x, const float* delta, int nsplit, int64_t split_stride, const float* w,
                        int rows, int D, float eps, const Act16* a, hipStream_t s, const int32_t* pick = nullptr,
                        int src_rows = 0);
-// inv[r] = the RMSNorm factor of row r < rows (RowNorm::inv of the consumers).
+// inv[r] = the RMSNorm factor of row r < rows (the consumers' RowNorm::ssq, nblk = 0).
 int launch_row_inv(float* inv, const RowNorm& rn, int rows, hipStream_t s);
 int launch_silu_act(float* y, const float* gate, const float* up, int rows, int H, int nsplit,
                     int64_t split_stride, int64_t ld, const Act16* a, const RowNorm& rn, hipStream_t s);
