@@ -17,6 +17,7 @@
 
 #include "launch.h"
 #include "act16.h"
+#include "attn_runs.h"
 #include "lanes.h"
 #include "rowops.h"
 #include "mfma.h"
@@ -362,20 +363,16 @@ __device__ __forceinline__ void attn_rope_prologue(const AttnRope& fr, int t, in
 // Partials (chunk max m, sum l, unnormalised output) as attn_block_kernel.
 // With ROPE the unit first runs attn_rope_prologue (q from LDS afterwards).
 template <int HD, int G, typename KVT, bool ROPE>
-__device__ __forceinline__ void attn_dec_body(const float* q, const KVT* Kp, const KVT* Vp, const int32_t* pairs,
-                                              int Hq, int64_t head_stride, int nch_max, float* po, float* pml,
-                                              const AttnRope& fr, int Hkv) {
+__device__ __forceinline__ void attn_dec_body(const float* q, const KVT* Kp, const KVT* Vp, const AttnUnit& un,
+                                              int h, int Hq, int64_t head_stride, int nch_max, float* po,
+                                              float* pml, const AttnRope& fr, int Hkv) {
     constexpr int NV = HD / 32;
     constexpr int LPR = HD / 4;
     constexpr int KPI = 64 / LPR;
     __shared__ float sp[G][ATT_CHUNK];
     __shared__ float4 sred[4][G][LPR];
     __shared__ float s_q[ROPE ? G : 1][ROPE ? HD : 1];
-    // work unit blockIdx.x of the (token, chunk) list that attn_pairs_kernel
-    // wrote; the units past its count are the grid's empty tail
-    const AttnUnit un = attn_unit(pairs, blockIdx.x);
-    if ((int)blockIdx.x >= un.n) return;
-    const int c = un.c, h = blockIdx.z, t = un.t, p = un.p;
+    const int c = un.c, t = un.t, p = un.p;
     const int k0 = c * ATT_CHUNK;
     if (k0 > p) return;                            // merge never reads chunks past a token's end
     const int nk = min(p + 1 - k0, ATT_CHUNK);
@@ -494,7 +491,11 @@ __global__ __launch_bounds__(ATT_THREADS) void attn_dec_kernel(
     const int32_t* __restrict__ dec_t0, const int32_t* __restrict__ tok2seq, const int32_t* __restrict__ tok_pos,
     const int64_t* __restrict__ kv_base, int Hq, int64_t head_stride, int nch_max, float* __restrict__ po,
     float* __restrict__ pml, const int32_t* __restrict__ pairs) {
-    attn_dec_body<HD, G, KVT, false>(q, Kp, Vp, pairs, Hq, head_stride, nch_max, po, pml, AttnRope{}, 0);
+    // work unit blockIdx.x of the (token, chunk) list that attn_pairs_kernel
+    // wrote; the units past its count are the grid's empty tail
+    const AttnUnit un = attn_unit(pairs, blockIdx.x);
+    if ((int)blockIdx.x >= un.n) return;
+    attn_dec_body<HD, G, KVT, false>(q, Kp, Vp, un, blockIdx.z, Hq, head_stride, nch_max, po, pml, AttnRope{}, 0);
 }
 
 // The phased unit with the rotation and KV append of the step's tokens (one
@@ -504,7 +505,33 @@ template <int HD, int G, typename KVT>
 __global__ __launch_bounds__(ATT_THREADS) void attn_dec_phased_rope_kernel(
     const KVT* Kp, const KVT* Vp, int Hq, int Hkv, int64_t head_stride, int nch_max, float* __restrict__ po,
     float* __restrict__ pml, const int32_t* __restrict__ pairs, AttnRope fr) {
-    attn_dec_body<HD, G, KVT, true>(nullptr, Kp, Vp, pairs, Hq, head_stride, nch_max, po, pml, fr, Hkv);
+    const AttnUnit un = attn_unit(pairs, blockIdx.x);
+    if ((int)blockIdx.x >= un.n) return;
+    attn_dec_body<HD, G, KVT, true>(nullptr, Kp, Vp, un, blockIdx.z, Hq, head_stride, nch_max, po, pml, fr, Hkv);
+}
+
+// Large calls over f32 caches: workgroup 0 lists the units of the run kernel
+// (k_attn_run.hip), the others run the tokens that kernel does not take,
+// workgroup 1 + (i * cx + x) * Hkv + h chunks x, x + cx, ... of token i and
+// kv head h.
+template <int HD, int G>
+__global__ __launch_bounds__(ATT_THREADS) void attn_single_kernel(
+    const float* __restrict__ q, const float* __restrict__ Kp, const float* __restrict__ Vp, RunTokens tk, int Hq,
+    int Hkv, int64_t head_stride, int nch_max, int cx, float* __restrict__ po, float* __restrict__ pml,
+    int32_t* __restrict__ list) {
+    if (blockIdx.x == 0) {
+        arn_build(tk, nch_max, arn_tokens(G), list);
+        return;
+    }
+    const uint32_t u = blockIdx.x - 1, r = u / Hkv;
+    const int i = r / cx;
+    if (!arn_single(tk, i)) return;
+    AttnUnit un{0, i, 0, tk.pos[i], tk.kv_base[tk.seq[i]]};
+    const int nc = min((un.p + ATT_CHUNK) / ATT_CHUNK, nch_max);
+    for (un.c = r % cx; un.c < nc; un.c += cx) {
+        attn_dec_body<HD, G, float, false>(q, Kp, Vp, un, u % Hkv, Hq, head_stride, nch_max, po, pml, AttnRope{}, 0);
+        __syncthreads();
+    }
 }
 
 // Decode work unit (one query token per sequence): (key chunk, token, kv
@@ -1173,6 +1200,28 @@ static bool runs_kernel(int HD, int n_dec, bool kv_f16) {
     return wave_kernel() && n_dec > ATT_WAVE_MAX_TOKENS && !kv_f16 && (HD == 32 || HD == 64 || HD == 128);
 }
 
+// Workgroups per token and kv head: as many as make a few thousand in all.
+constexpr int ATT_SINGLE_GRID = 8192;
+
+template <int HD>
+static int launch_single_hd(int G, hipStream_t s, const AttnArgs& a, const RunTokens& tk, int Hkv, int32_t* list) {
+    const int64_t pairs = (int64_t)tk.n * Hkv;
+    const int cx = (int)std::min<int64_t>(a.nch_max, (ATT_SINGLE_GRID + pairs - 1) / pairs);
+    const dim3 grid((unsigned)(1 + pairs * cx));
+    const float *Kp = (const float*)a.Kp, *Vp = (const float*)a.Vp;
+    switch (G) {
+        case 1: SH_LAUNCH(a.ev0, nullptr, (attn_single_kernel<HD, 1>), grid, dim3(ATT_THREADS), 0, s, a.q, Kp, Vp, tk,
+                          a.Hq, Hkv, a.head_stride, a.nch_max, cx, a.po, a.pml, list); return 0;
+        case 2: SH_LAUNCH(a.ev0, nullptr, (attn_single_kernel<HD, 2>), grid, dim3(ATT_THREADS), 0, s, a.q, Kp, Vp, tk,
+                          a.Hq, Hkv, a.head_stride, a.nch_max, cx, a.po, a.pml, list); return 0;
+        case 4: SH_LAUNCH(a.ev0, nullptr, (attn_single_kernel<HD, 4>), grid, dim3(ATT_THREADS), 0, s, a.q, Kp, Vp, tk,
+                          a.Hq, Hkv, a.head_stride, a.nch_max, cx, a.po, a.pml, list); return 0;
+        case 8: SH_LAUNCH(a.ev0, nullptr, (attn_single_kernel<HD, 8>), grid, dim3(ATT_THREADS), 0, s, a.q, Kp, Vp, tk,
+                          a.Hq, Hkv, a.head_stride, a.nch_max, cx, a.po, a.pml, list); return 0;
+        default: return -5;
+    }
+}
+
 template <int HD, int G, typename KVT>
 static void launch_dec_t(dim3 grid, hipStream_t s, const AttnArgs& a) {
     const KVT* Kp = (const KVT*)a.Kp;
@@ -1246,10 +1295,18 @@ int launch_attention_blocks(float* out, const float* q, const void* Kp, const vo
             rc = launch_attention_prompt(q, (const float*)Kp, (const float*)Vp, tok2seq, tok_pos, kv_base, pre_t0,
                                          pre_n, n_pre, Hq, Hkv, HD, head_stride, nch_max, po, pml, s, a.ev0);
             if (rc) return rc;
-        } else if (runs_kernel(HD, n_dec, kv_f16) && !prefill && !pairs_ready && head_stride % 4 == 0 &&
+        } else if (runs_kernel(HD, n_dec, kv_f16) && !prefill && !pairs_ready && !dec_t0 && head_stride % 4 == 0 &&
                    (((uintptr_t)q | (uintptr_t)Kp | (uintptr_t)Vp) & 15) == 0) {
-            rc = launch_attention_runs(q, (const float*)Kp, (const float*)Vp, tok2seq, tok_pos, kv_base, dec_t0,
-                                       n_dec, Hq, Hkv, HD, head_stride, nch_max, po, pml, pairs, s, a.ev0);
+            // `pairs` holds the run kernel's list here: as many entries at most
+            const RunTokens tk{tok2seq, tok_pos, kv_base, n_dec};
+            rc = HD == 128 ? launch_single_hd<128>(G, s, a, tk, Hkv, pairs)
+                           : (HD == 64 ? launch_single_hd<64>(G, s, a, tk, Hkv, pairs)
+                                       : launch_single_hd<32>(G, s, a, tk, Hkv, pairs));
+            if (rc == 0) {
+                SH_CHECK_LAUNCH();
+                rc = launch_attention_runs(q, (const float*)Kp, (const float*)Vp, n_dec, Hq, Hkv, HD, head_stride,
+                                           nch_max, po, pml, pairs, s);
+            }
         } else if (!prefill && (HD == 32 || HD == 64 || HD == 128)) {
             if (!pairs_ready) {
                 SH_LAUNCH(a.ev0, nullptr, attn_pairs_kernel, dim3(1), dim3(1024), 0, s, dec_t0, n_dec, tok_pos,

@@ -3,11 +3,11 @@
 //
 // attention_ragged takes its tokens one by one (sequence and position per
 // token, in device memory), so a prompt chunk arrives as tokens that follow
-// each other in one sequence.  attn_runs_kernel finds these runs on the
-// device and cuts them into units of up to 16 / G tokens (16 query rows with
-// the G heads of a group) times a chunk of 256 keys; attn_run_kernel streams
-// each unit's K and V rows once for all its rows.  A token that follows no
-// other is a unit of its own.
+// each other in one sequence.  attn_single_kernel (k_attn.hip) finds these
+// runs on the device and cuts them into units of up to 16 / G tokens (16 query
+// rows with the G heads of a group) times a chunk of 256 keys; attn_run_kernel
+// streams each unit's K and V rows once for all its rows.  A token that
+// follows no other is a unit of its own.
 //
 // A unit's four waves own up to 64 keys each.  Scores are S^T = K Q^T (16 keys x 16
 // rows per MFMA tile, 4 dims a step): a lane holds scores of one row, keys
@@ -34,94 +34,12 @@
 #include <cfloat>
 
 #include "launch.h"
-#include "lanes.h"
+#include "attn_runs.h"
 #include "mfma.h"
 
 namespace slate_hip {
 
-constexpr int ARN_CHUNK = 256;       // keys per unit: the merge kernel's chunk
 constexpr int ARN_KW = 64;           // keys per wave, at most
-constexpr int ARN_ROWS = 16;         // query rows per unit
-constexpr int ARN_LIST = 1024;       // threads of the list kernel
-
-__host__ __device__ constexpr int arn_tokens(int G) { return ARN_ROWS / G; }
-
-// Inclusive scan over the workgroup's 1024 threads (sum, or maximum).
-template <bool MAX>
-__device__ __forceinline__ int wg_scan(int v, int* s_w) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(v, o, 64);
-        if (lane >= o) v = MAX ? max(v, u) : v + u;
-    }
-    if (lane == 63) s_w[wv] = v;
-    __syncthreads();
-    int b = MAX ? INT32_MIN : 0;
-    for (int w = 0; w < wv; ++w) b = MAX ? max(b, s_w[w]) : b + s_w[w];
-    __syncthreads();
-    return MAX ? max(v, b) : v + b;
-}
-
-// Unit list: list[0] = count, then from list + 4 one int4 per unit {first
-// token * 65536 + chunk, its position, low word of the K/V base, next 24
-// bits of the base + (tokens << 24)}.  A run is a series of entries whose
-// tokens follow each other in memory and, at positions one apart, in one
-// sequence; entries 1024 apart are never joined.  At most one unit per entry
-// and chunk.
-__global__ __launch_bounds__(ARN_LIST) void attn_runs_kernel(const int32_t* __restrict__ dec_t0, int n_dec,
-                                                             const int32_t* __restrict__ tok_pos,
-                                                             const int32_t* __restrict__ tok2seq,
-                                                             const int64_t* __restrict__ kv_base, int nch_max,
-                                                             int tb, int32_t* __restrict__ list) {
-    __shared__ int s_w[ARN_LIST / 64];
-    __shared__ int s_tot;
-    __shared__ int s_t[ARN_LIST], s_p[ARN_LIST], s_s[ARN_LIST];
-    __shared__ unsigned char s_start[ARN_LIST];
-    const int tid = threadIdx.x;
-    int4* units = (int4*)(list + 4);
-    int base = 0;
-    for (int i0 = 0; i0 < n_dec; i0 += ARN_LIST) {
-        const int i = i0 + tid;
-        int t = 0, p = 0, sq = 0;
-        int64_t kvb = 0;
-        if (i < n_dec) {
-            t = dec_t0 ? dec_t0[i] : i;
-            p = tok_pos[t];
-            sq = tok2seq[t];
-            kvb = kv_base[sq];
-        }
-        s_t[tid] = t;
-        s_p[tid] = p;
-        s_s[tid] = sq;
-        __syncthreads();
-        const bool start = tid == 0 || i >= n_dec || s_t[tid - 1] != t - 1 || s_s[tid - 1] != sq ||
-                           s_p[tid - 1] != p - 1;
-        s_start[tid] = start;
-        const int first = wg_scan<true>(start ? tid : 0, s_w);    // (its barriers publish s_start too)
-        int n = 0, nc = 0;
-        if (i < n_dec && (tid - first) % tb == 0) {
-            n = 1;
-            while (n < tb && tid + n < ARN_LIST && !s_start[tid + n]) ++n;
-            nc = max(0, min((p + n - 1 + ARN_CHUNK) / ARN_CHUNK, nch_max));
-        }
-        const int end = wg_scan<false>(nc, s_w);
-        for (int c = 0; c < nc; ++c)
-            units[base + end - nc + c] =
-                make_int4(t * 65536 + c, p, (int)(uint32_t)((uint64_t)kvb & 0xffffffffu),
-                          (int)(((uint32_t)((uint64_t)kvb >> 32) & 0xffffffu) | ((uint32_t)n << 24)));
-        if (tid == ARN_LIST - 1) s_tot = end;
-        __syncthreads();
-        base += s_tot;
-        __syncthreads();
-    }
-    if (tid == 0) list[0] = base;
-}
-
-struct RunUnit {
-    int t0, n, p0, c;        // first token, tokens, first position, key chunk
-    int64_t kv;              // first key of the chunk in the K and V pools, this kv head
-};
 
 template <int HD>
 struct RunGeom {
@@ -150,8 +68,9 @@ __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)"
 
 template <int HD, int G>
 __device__ __forceinline__ void attn_run_unit(const float* q, const float* Kp, const float* Vp, const RunUnit& un,
-                                              int h, int Hq, int nch_max, float* __restrict__ po,
-                                              float* __restrict__ pml, float* s_o, float* s_q) {
+                                              int h, int Hq, int64_t head_stride, int nch_max,
+                                              float* __restrict__ po, float* __restrict__ pml, float* s_o,
+                                              float* s_q) {
     using Geo = RunGeom<HD>;
     constexpr int NT = Geo::NT, VW = Geo::VW, NB = Geo::NB, CPR = Geo::CPR, KT = ARN_KW / 16, R = ARN_ROWS;
     typedef float vf_t __attribute__((ext_vector_type(VW)));
@@ -167,8 +86,9 @@ __device__ __forceinline__ void attn_run_unit(const float* q, const float* Kp, c
     const int kn = min(nk - kw0, kw);                       // the wave's keys
     const bool active = kn > 0;
     const float scale = 1.0f / sqrtf((float)HD);
-    const float* Kh = Kp + un.kv;
-    const float* Vh = Vp + un.kv;
+    const int64_t key0 = un.kvb + (int64_t)h * head_stride + (int64_t)k0 * HD;   // the chunk's first key
+    const float* Kh = Kp + key0;
+    const float* Vh = Vp + key0;
     float* so = s_o + wv * Geo::WAVE;
     // ---- the unit's query rows (row r: token r / G, head r % G; rows past
     // its tokens repeat the last one), and the wave's first K tile
@@ -401,15 +321,8 @@ __global__ __launch_bounds__(256, HD == 128 ? 3 : 4) void attn_run_kernel(const 
     __shared__ __attribute__((aligned(16))) float s_q[ARN_ROWS * HD];
     const int h = blockIdx.x, total = list[0];
     for (int u = blockIdx.y; u < total; u += gridDim.y) {
-        const int4 d = ((const int4*)(list + 4))[u];
-        RunUnit un;
-        un.t0 = d.x >> 16;
-        un.c = d.x & 0xffff;
-        un.p0 = d.y;
-        un.n = (int)((uint32_t)d.w >> 24);
-        const int64_t kvb = ((int64_t)(((uint64_t)(uint32_t)d.w << 32) | (uint32_t)d.z) << 8) >> 8;
-        un.kv = kvb + (int64_t)h * head_stride + (int64_t)un.c * ARN_CHUNK * HD;
-        attn_run_unit<HD, G>(q, Kp, Vp, un, h, Hq, nch_max, po, pml, s_o, s_q);
+        const RunUnit un = arn_unpack(((const int4*)(list + 4))[u]);
+        attn_run_unit<HD, G>(q, Kp, Vp, un, h, Hq, head_stride, nch_max, po, pml, s_o, s_q);
         __syncthreads();
     }
 }
@@ -417,39 +330,32 @@ __global__ __launch_bounds__(256, HD == 128 ? 3 : 4) void attn_run_kernel(const 
 constexpr int ARN_GRID = 4096;
 
 template <int HD>
-static int launch_run_hd(int G, dim3 grid, hipStream_t s, hipEvent_t ev0, const float* q, const float* Kp,
-                         const float* Vp, int Hq, int64_t head_stride, int nch_max, float* po, float* pml,
-                         const int32_t* list) {
+static int launch_run_hd(int G, dim3 grid, hipStream_t s, const float* q, const float* Kp, const float* Vp, int Hq,
+                         int64_t head_stride, int nch_max, float* po, float* pml, const int32_t* list) {
     switch (G) {
-        case 1: SH_LAUNCH(ev0, nullptr, (attn_run_kernel<HD, 1>), grid, dim3(256), 0, s, q, Kp, Vp, Hq,
-                          head_stride, nch_max, po, pml, list); return 0;
-        case 2: SH_LAUNCH(ev0, nullptr, (attn_run_kernel<HD, 2>), grid, dim3(256), 0, s, q, Kp, Vp, Hq,
-                          head_stride, nch_max, po, pml, list); return 0;
-        case 4: SH_LAUNCH(ev0, nullptr, (attn_run_kernel<HD, 4>), grid, dim3(256), 0, s, q, Kp, Vp, Hq,
-                          head_stride, nch_max, po, pml, list); return 0;
-        case 8: SH_LAUNCH(ev0, nullptr, (attn_run_kernel<HD, 8>), grid, dim3(256), 0, s, q, Kp, Vp, Hq,
-                          head_stride, nch_max, po, pml, list); return 0;
+        case 1: hipLaunchKernelGGL((attn_run_kernel<HD, 1>), grid, dim3(256), 0, s, q, Kp, Vp, Hq, head_stride,
+                                   nch_max, po, pml, list); return 0;
+        case 2: hipLaunchKernelGGL((attn_run_kernel<HD, 2>), grid, dim3(256), 0, s, q, Kp, Vp, Hq, head_stride,
+                                   nch_max, po, pml, list); return 0;
+        case 4: hipLaunchKernelGGL((attn_run_kernel<HD, 4>), grid, dim3(256), 0, s, q, Kp, Vp, Hq, head_stride,
+                                   nch_max, po, pml, list); return 0;
+        case 8: hipLaunchKernelGGL((attn_run_kernel<HD, 8>), grid, dim3(256), 0, s, q, Kp, Vp, Hq, head_stride,
+                                   nch_max, po, pml, list); return 0;
         default: return -5;
     }
 }
 
-// List and partials of n_dec tokens (list: the storage of the decode unit
-// list, one int4 per token and chunk).
-int launch_attention_runs(const float* q, const float* Kp, const float* Vp, const int32_t* tok2seq,
-                          const int32_t* tok_pos, const int64_t* kv_base, const int32_t* dec_t0, int n_dec, int Hq,
-                          int Hkv, int HD, int64_t head_stride, int nch_max, float* po, float* pml, int32_t* list,
-                          hipStream_t s, hipEvent_t ev_start) {
+// Partials of the units in `list` (at most one per token and chunk of n tokens).
+int launch_attention_runs(const float* q, const float* Kp, const float* Vp, int n, int Hq, int Hkv, int HD,
+                          int64_t head_stride, int nch_max, float* po, float* pml, const int32_t* list,
+                          hipStream_t s) {
     const int G = Hq / Hkv;
-    if (attn_chunk_size() != ARN_CHUNK || (G != 1 && G != 2 && G != 4 && G != 8)) return -5;
-    SH_LAUNCH(ev_start, nullptr, attn_runs_kernel, dim3(1), dim3(ARN_LIST), 0, s, dec_t0, n_dec, tok_pos, tok2seq,
-              kv_base, nch_max, arn_tokens(G), list);
-    SH_CHECK_LAUNCH();
-    const dim3 grid(Hkv, (unsigned)std::min<int64_t>(std::max(1, ARN_GRID / Hkv), (int64_t)n_dec * nch_max));
-    const int rc =
-        HD == 128 ? launch_run_hd<128>(G, grid, s, nullptr, q, Kp, Vp, Hq, head_stride, nch_max, po, pml, list)
-        : HD == 64 ? launch_run_hd<64>(G, grid, s, nullptr, q, Kp, Vp, Hq, head_stride, nch_max, po, pml, list)
-        : HD == 32 ? launch_run_hd<32>(G, grid, s, nullptr, q, Kp, Vp, Hq, head_stride, nch_max, po, pml, list)
-                   : -5;
+    if (attn_chunk_size() != ARN_CHUNK) return -5;
+    const dim3 grid(Hkv, (unsigned)std::min<int64_t>(std::max(1, ARN_GRID / Hkv), (int64_t)n * nch_max));
+    const int rc = HD == 128 ? launch_run_hd<128>(G, grid, s, q, Kp, Vp, Hq, head_stride, nch_max, po, pml, list)
+                   : HD == 64 ? launch_run_hd<64>(G, grid, s, q, Kp, Vp, Hq, head_stride, nch_max, po, pml, list)
+                   : HD == 32 ? launch_run_hd<32>(G, grid, s, q, Kp, Vp, Hq, head_stride, nch_max, po, pml, list)
+                              : -5;
     if (rc) return rc;
     SH_CHECK_LAUNCH();
     return 0;

@@ -128,14 +128,12 @@ int launch_attention_prompt(const float* q, const float* Kp, const float* Vp, co
                             const int32_t* blk_n, int n_blk, int Hq, int Hkv, int HD, int64_t head_stride,
                             int nch_max, float* po, float* pml, hipStream_t s, hipEvent_t ev0);
 
-// k_attn_run.hip: the partials of n_dec query tokens (dec_t0, or 0 .. n_dec-1)
-// over f32 caches, runs of consecutive tokens of one sequence found on the
-// device and sharing their K/V rows.  list: storage of the decode unit list.
+// k_attn_run.hip: the partials of the listed units (attn_runs.h) of n tokens
+// over f32 caches, a unit's tokens sharing their K/V rows.
 // -5 for a head_dim / group it does not cover (32, 64, 128; 1, 2, 4, 8).
-int launch_attention_runs(const float* q, const float* Kp, const float* Vp, const int32_t* tok2seq,
-                          const int32_t* tok_pos, const int64_t* kv_base, const int32_t* dec_t0, int n_dec, int Hq,
-                          int Hkv, int HD, int64_t head_stride, int nch_max, float* po, float* pml, int32_t* list,
-                          hipStream_t s, hipEvent_t ev_start);
+int launch_attention_runs(const float* q, const float* Kp, const float* Vp, int n, int Hq, int Hkv, int HD,
+                          int64_t head_stride, int nch_max, float* po, float* pml, const int32_t* list,
+                          hipStream_t s);
 
 // k_synth.hip
 int launch_synth_f32(float* dst, int64_t n, uint64_t seed, float std, float fill, hipStream_t s);

@@ -319,3 +319,52 @@ def test_attention_runs(hip, hd, Hq, Hkv, order):
         else:
             # (the last tokens of a run take the exact path of their unit)
             assert np.allclose(again[t], got[t], rtol=0, atol=64 * EPS * 8), (t, tok[t])
+
+
+def _check_attention(hip, rng, tok, hd, Hq, Hkv, stride, offs, off=(0, 0, 0)):
+    """attention_ragged of tokens (sequence, position) against float64: kv
+    heads `stride` floats apart, sequence b's base offs[b] floats off, the
+    pointers of q, K and V off[i] floats off 16 bytes."""
+    S, nslot, T = 768, len(offs), len(tok)
+    seq = np.array([s for s, _ in tok], np.int32)
+    pos = np.array([p for _, p in tok], np.int32)
+    base = np.arange(nslot, dtype=np.int64) * (Hkv * stride + 4) + np.array(offs)
+    pool = int(base[-1]) + Hkv * stride + 4
+    K, V = (rng.normal(0, 1, pool).astype(np.float32) for _ in range(2))
+    q = rng.normal(0, 1, (T, Hq, hd)).astype(np.float32)
+    bufs = []
+    for a, o in zip((q, K, V), off):
+        bufs.append(DB((a.size + 4) * 4))
+        bufs[-1].upload(np.concatenate([np.zeros(o, np.float32), a.reshape(-1), np.zeros(4 - o, np.float32)]))
+    out = DB((T * Hq * hd + 64) * 4)
+    out.upload(np.full(T * Hq * hd + 64, 7.0, np.float32))
+    check(hip.lib.slate_hip_attention_ragged(
+        out.p, *[b.ptr + 4 * o for b, o in zip(bufs, off)], DB.from_array(seq).p, DB.from_array(pos).p,
+        DB.from_array(base).p, T, Hq, Hkv, hd, stride, S), "attention_ragged")
+    got = host(out, (T * Hq * hd + 64,))
+    assert np.all(got[T * Hq * hd:] == 7.0)
+    got = got[:T * Hq * hd].reshape(T, Hkv, Hq // Hkv, hd)
+    q6 = q.astype(np.float64).reshape(got.shape)
+    for t in range(T):
+        L = pos[t] + 1
+        for h in range(Hkv):
+            b = int(base[seq[t]]) + h * stride
+            k, v = (a[b:b + L * hd].astype(np.float64).reshape(L, hd) for a in (K, V))
+            s = q6[t, h] @ k.T / np.sqrt(hd)
+            mag = (np.abs(q6[t, h]) @ np.abs(k).T).max() / np.sqrt(hd)
+            p = np.exp(s - s.max(-1, keepdims=True))
+            p /= p.sum(-1, keepdims=True)
+            # (the bound of test_attention_runs)
+            bound = (2 * (hd + 8) * EPS * mag + (min(L, 256) + 64) * EPS) * (p @ np.abs(v))
+            assert np.all(np.abs(got[t, h] - p @ v) <= bound), (t, tok[t], h)
+
+
+# More than 64 tokens: rows that start on 16 bytes only in some sequences
+# (kv_base takes any offset), and q, K, V or the heads off 16 bytes.
+@pytest.mark.parametrize("hd,Hq,Hkv", [(128, 8, 2), (64, 8, 8), (32, 8, 1)])
+@pytest.mark.parametrize("form", ["base", "q", "K", "V", "stride"])
+def test_attention_of_unaligned_rows(hip, hd, Hq, Hkv, form):
+    offs = (1, 0, 3, 0, 2, 0, 1) if form == "base" else (0,) * 7
+    off = {"q": (1, 0, 0), "K": (0, 3, 0), "V": (0, 0, 2)}.get(form, (0, 0, 0))
+    _check_attention(hip, np.random.default_rng(hd + len(form)), _ragged_case(None, "joined"), hd, Hq, Hkv,
+                     768 * hd + (1 if form == "stride" else 0), offs, off)
