@@ -362,7 +362,8 @@ __device__ __forceinline__ void attn_rope_prologue(const AttnRope& fr, int t, in
 //           probabilities broadcast from LDS, reduced over lanes and waves.
 // Partials (chunk max m, sum l, unnormalised output) as attn_block_kernel.
 // With ROPE the unit first runs attn_rope_prologue (q from LDS afterwards).
-template <int HD, int G, typename KVT, bool ROPE>
+// LOOP: the caller runs unit after unit.
+template <int HD, int G, typename KVT, bool ROPE, bool LOOP = false>
 __device__ __forceinline__ void attn_dec_body(const float* q, const KVT* Kp, const KVT* Vp, const AttnUnit& un,
                                               int h, int Hq, int64_t head_stride, int nch_max, float* po,
                                               float* pml, const AttnRope& fr, int Hkv) {
@@ -377,7 +378,9 @@ __device__ __forceinline__ void attn_dec_body(const float* q, const KVT* Kp, con
     if (k0 > p) return;                            // merge never reads chunks past a token's end
     const int nk = min(p + 1 - k0, ATT_CHUNK);
     const int nkp = (nk + 31) & ~31;               // rounds of 32 keys (multiple of 4 * KPI)
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    int tid = threadIdx.x;
+    if constexpr (LOOP) asm volatile("" : "+v"(tid));   // offsets computed per unit, not held from unit to unit
+    const int lane = tid & 63, wv = tid >> 6;
     const int lg = lane >> 3, ls = lane & 7;
     const float scale = 1.0f / sqrtf((float)HD);
     const int64_t base = un.kvb + (int64_t)h * head_stride + (int64_t)k0 * HD;
@@ -511,25 +514,42 @@ __global__ __launch_bounds__(ATT_THREADS) void attn_dec_phased_rope_kernel(
 }
 
 // Large calls over f32 caches: workgroup 0 lists the units of the run kernel
-// (k_attn_run.hip), the others run the tokens that kernel does not take,
-// workgroup 1 + (i * cx + x) * Hkv + h chunks x, x + cx, ... of token i and
-// kv head h.
+// (k_attn_run.hip), the others share the (token, chunk, kv head) triples of the
+// passes that kernel does not take (attn_runs.h).  Each numbers them for
+// itself, so that no list kernel has to run first.
+//
+// Bound by the latency of a unit's loads and barriers at short contexts, by
+// HBM at long ones.  Against every call of this size through the run kernel
+// (in brackets: the list and phased kernels): 128 lone tokens at ~60 keys, 32
+// q / 8 kv heads of 128, 28.2 -> 21.2 us (20.9); at ~16 keys, 32 kv heads, 41.8
+// -> 22.2 (20.8); 60 decode tokens at ~500 keys and a chunk of 5, 16 q / 4 kv
+// heads of 64, 22.5 -> 19.9 (20.0).  Above about 300 tokens of at most 60 keys
+// the shares' lockstep costs up to a quarter against the phased kernel
+// (512 at ~16 keys: 47.4 -> 37.1, 29.8).
 template <int HD, int G>
-__global__ __launch_bounds__(ATT_THREADS) void attn_single_kernel(
+__global__ __launch_bounds__(ATT_THREADS) void attn_token_kernel(
     const float* __restrict__ q, const float* __restrict__ Kp, const float* __restrict__ Vp, RunTokens tk, int Hq,
-    int Hkv, int64_t head_stride, int nch_max, int cx, float* __restrict__ po, float* __restrict__ pml,
+    int Hkv, int64_t head_stride, int nch_max, float* __restrict__ po, float* __restrict__ pml,
     int32_t* __restrict__ list) {
     if (blockIdx.x == 0) {
-        arn_build(tk, nch_max, arn_tokens(G), list);
+        arn_build(tk, nch_max, arn_tokens(G), HD, list);
         return;
     }
-    const uint32_t u = blockIdx.x - 1, r = u / Hkv;
-    const int i = r / cx;
-    if (!arn_single(tk, i)) return;
-    AttnUnit un{0, i, 0, tk.pos[i], tk.kv_base[tk.seq[i]]};
-    const int nc = min((un.p + ATT_CHUNK) / ATT_CHUNK, nch_max);
-    for (un.c = r % cx; un.c < nc; un.c += cx) {
-        attn_dec_body<HD, G, float, false>(q, Kp, Vp, un, u % Hkv, Hq, head_stride, nch_max, po, pml, AttnRope{}, 0);
+    __shared__ TokenPass s_pass;
+    int64_t u = blockIdx.x - 1;
+    for (int i0 = 0; i0 < tk.n; i0 += ARN_PASS) {
+        const int64_t items = (int64_t)s_pass.number(tk, i0, nch_max, arn_tokens(G), HD) * Hkv;
+        for (; u < items; u += gridDim.x - 1) {
+            AttnUnit un{};
+            s_pass.pair((int)(u / Hkv), un.t, un.c);
+            un.t += i0;
+            un.p = tk.pos[un.t];
+            un.kvb = tk.kv_base[tk.seq[un.t]];
+            attn_dec_body<HD, G, float, false, true>(q, Kp, Vp, un, (int)(u % Hkv), Hq, head_stride, nch_max, po, pml,
+                                                     AttnRope{}, 0);
+            __syncthreads();
+        }
+        u -= items;
         __syncthreads();
     }
 }
@@ -1190,34 +1210,36 @@ static bool wave_kernel() { return knobs().attn_wave != 0; }
 
 // The wave kernel where its query slices and accumulators fit the registers
 // and the launch is a decode batch (a few query tokens, K/V streamed from
-// HBM); prompt tokens, whose K/V re-reads hit L2, run the phased kernel at
-// its higher occupancy.
+// HBM); larger launches, whose K/V re-reads hit L2, run the phased kernel at
+// its higher occupancy, and f32 calls of the C ABI the pair of kernels below.
 constexpr int ATT_WAVE_MAX_TOKENS = 64;
 // Past the decode batches prompt chunks are among the tokens, and runs of
 // them share their K/V rows (65 to 71 tokens with two to four chunks: 1.1 to
-// 1.7x; k_attn_run.hip).
+// 1.7x; k_attn_run.hip) where that saves enough (arn_shared).
 static bool runs_kernel(int HD, int n_dec, bool kv_f16) {
     return wave_kernel() && n_dec > ATT_WAVE_MAX_TOKENS && !kv_f16 && (HD == 32 || HD == 64 || HD == 128);
 }
 
-// Workgroups per token and kv head: as many as make a few thousand in all.
-constexpr int ATT_SINGLE_GRID = 8192;
+static int device_cus();
+
+// As many workgroups as the device holds at once: each numbers the call's
+// pairs before its first triple, and a second round would do so again.
+template <int HD, int G>
+static void launch_token(hipStream_t s, const AttnArgs& a, const RunTokens& tk, int Hkv, int32_t* list) {
+    constexpr int FIT = G * HD > 512 ? 2 : (G * HD > 256 ? 4 : (G * HD > 128 ? 5 : 6));   // by their registers
+    static const int cus = device_cus();
+    const dim3 grid((unsigned)(1 + std::min<int64_t>((int64_t)tk.n * a.nch_max * Hkv, FIT * cus)));
+    SH_LAUNCH(a.ev0, nullptr, (attn_token_kernel<HD, G>), grid, dim3(ATT_THREADS), 0, s, a.q, (const float*)a.Kp,
+              (const float*)a.Vp, tk, a.Hq, Hkv, a.head_stride, a.nch_max, a.po, a.pml, list);
+}
 
 template <int HD>
-static int launch_single_hd(int G, hipStream_t s, const AttnArgs& a, const RunTokens& tk, int Hkv, int32_t* list) {
-    const int64_t pairs = (int64_t)tk.n * Hkv;
-    const int cx = (int)std::min<int64_t>(a.nch_max, (ATT_SINGLE_GRID + pairs - 1) / pairs);
-    const dim3 grid((unsigned)(1 + pairs * cx));
-    const float *Kp = (const float*)a.Kp, *Vp = (const float*)a.Vp;
+static int launch_token_hd(int G, hipStream_t s, const AttnArgs& a, const RunTokens& tk, int Hkv, int32_t* list) {
     switch (G) {
-        case 1: SH_LAUNCH(a.ev0, nullptr, (attn_single_kernel<HD, 1>), grid, dim3(ATT_THREADS), 0, s, a.q, Kp, Vp, tk,
-                          a.Hq, Hkv, a.head_stride, a.nch_max, cx, a.po, a.pml, list); return 0;
-        case 2: SH_LAUNCH(a.ev0, nullptr, (attn_single_kernel<HD, 2>), grid, dim3(ATT_THREADS), 0, s, a.q, Kp, Vp, tk,
-                          a.Hq, Hkv, a.head_stride, a.nch_max, cx, a.po, a.pml, list); return 0;
-        case 4: SH_LAUNCH(a.ev0, nullptr, (attn_single_kernel<HD, 4>), grid, dim3(ATT_THREADS), 0, s, a.q, Kp, Vp, tk,
-                          a.Hq, Hkv, a.head_stride, a.nch_max, cx, a.po, a.pml, list); return 0;
-        case 8: SH_LAUNCH(a.ev0, nullptr, (attn_single_kernel<HD, 8>), grid, dim3(ATT_THREADS), 0, s, a.q, Kp, Vp, tk,
-                          a.Hq, Hkv, a.head_stride, a.nch_max, cx, a.po, a.pml, list); return 0;
+        case 1: launch_token<HD, 1>(s, a, tk, Hkv, list); return 0;
+        case 2: launch_token<HD, 2>(s, a, tk, Hkv, list); return 0;
+        case 4: launch_token<HD, 4>(s, a, tk, Hkv, list); return 0;
+        case 8: launch_token<HD, 8>(s, a, tk, Hkv, list); return 0;
         default: return -5;
     }
 }
@@ -1299,9 +1321,9 @@ int launch_attention_blocks(float* out, const float* q, const void* Kp, const vo
                    (((uintptr_t)q | (uintptr_t)Kp | (uintptr_t)Vp) & 15) == 0) {
             // `pairs` holds the run kernel's list here: as many entries at most
             const RunTokens tk{tok2seq, tok_pos, kv_base, n_dec};
-            rc = HD == 128 ? launch_single_hd<128>(G, s, a, tk, Hkv, pairs)
-                           : (HD == 64 ? launch_single_hd<64>(G, s, a, tk, Hkv, pairs)
-                                       : launch_single_hd<32>(G, s, a, tk, Hkv, pairs));
+            rc = HD == 128 ? launch_token_hd<128>(G, s, a, tk, Hkv, pairs)
+                           : (HD == 64 ? launch_token_hd<64>(G, s, a, tk, Hkv, pairs)
+                                       : launch_token_hd<32>(G, s, a, tk, Hkv, pairs));
             if (rc == 0) {
                 SH_CHECK_LAUNCH();
                 rc = launch_attention_runs(q, (const float*)Kp, (const float*)Vp, n_dec, Hq, Hkv, HD, head_stride,

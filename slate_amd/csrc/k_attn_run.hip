@@ -3,7 +3,7 @@
 //
 // attention_ragged takes its tokens one by one (sequence and position per
 // token, in device memory), so a prompt chunk arrives as tokens that follow
-// each other in one sequence.  attn_single_kernel (k_attn.hip) finds these
+// each other in one sequence.  attn_token_kernel (k_attn.hip) finds these
 // runs on the device and cuts them into units of up to 16 / G tokens (16 query
 // rows with the G heads of a group) times a chunk of 256 keys; attn_run_kernel
 // streams each unit's K and V rows once for all its rows.  A token that
@@ -26,9 +26,9 @@
 // keys and three chunks of 121-172 tokens (32 q / 8 kv heads of 128), the
 // whole call: 139 us token by token, 89 here; 32 q and kv heads of 128, four
 // chunks of up to 98 tokens: 55 and 28 us; 16 q / 4 kv heads of 64, four of up
-// to 68 beside nine decode tokens: 32 and 23.  Lone tokens gain nothing (128
-// at ~300 keys 92 and 90 us, 300 at ~60 keys 23 and 25).  32 rows a unit halve the K/V
-// traffic but leave two waves a SIMD: 102 us.  Chains of four MFMAs fit 128
+// to 68 beside nine decode tokens: 32 and 23.  Lone tokens gain nothing, and
+// lose at short contexts: such calls go to the token kernel (attn_runs.h).  32
+// rows a unit halve the K/V traffic but leave two waves a SIMD: 102 us.  Chains of four MFMAs fit 128
 // registers (four waves; 86 us where these took 93), but round 3 to 10 % worse.
 #include <algorithm>
 #include <cfloat>

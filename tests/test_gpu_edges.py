@@ -368,3 +368,24 @@ def test_attention_of_unaligned_rows(hip, hd, Hq, Hkv, form):
     off = {"q": (1, 0, 0), "K": (0, 3, 0), "V": (0, 0, 2)}.get(form, (0, 0, 0))
     _check_attention(hip, np.random.default_rng(hd + len(form)), _ragged_case(None, "joined"), hd, Hq, Hkv,
                      768 * hd + (1 if form == "stride" else 0), offs, off)
+
+
+# More than 64 tokens that hardly share keys (each workgroup of the token kernel
+# numbers them for itself) and calls of several passes of 1024 tokens: all
+# alone, short and long; alone but for a pair; a pass alone, then runs that
+# begin before the pass does and end in it; an unaligned sequence in one pass.
+@pytest.mark.parametrize("hd,Hq,Hkv", [(128, 4, 1), (128, 2, 2), (64, 8, 1), (32, 6, 3)])
+@pytest.mark.parametrize("form", ["short", "long", "pair", "passes", "unaligned pass"])
+def test_attention_of_lone_tokens(hip, hd, Hq, Hkv, form):
+    rng = np.random.default_rng(hd * Hq + len(form))
+    offs = [0] * 7
+    tok = [(i % 6, int(p)) for i, p in enumerate(rng.integers(0, 700 if form == "long" else 90, 65))]
+    if form == "pair":
+        tok += [(6, 255), (6, 256)]
+    if form in ("passes", "unaligned pass"):
+        tok = [(i % 6, (37 * i) % 41) for i in range(1020)] + [(6, i) for i in range(200)]
+        tok += [(i % 3, 700 - i) for i in range(700)] + [(4, i) for i in range(228)]
+    if form == "unaligned pass":
+        offs[2] = 3
+        tok = tok[:1024] + [(6, 4 + i) for i in range(300)]
+    _check_attention(hip, rng, tok, hd, Hq, Hkv, 768 * hd, tuple(offs))
