@@ -206,6 +206,10 @@ __device__ __forceinline__ half8_t q4k_bop(const WTile& w, const WScale& c, int 
     return half8_t{p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
 }
 
+// Blocks of a decode split: where the engine's consumers add the splits, and
+// where a split sum does (dec_plan).
+constexpr int DEC_BPS_STEP = 8, DEC_BPS_OP = 4;
+
 // Decode kernel (NT = 1 or 2 16-row activation tiles: up to 32 rows).  A
 // workgroup of WAVES waves owns WAVES*R weight tiles (possibly spread over
 // up to three fused tensors) and one split of super-blocks.  The NT tiles'
@@ -228,6 +232,10 @@ __device__ __forceinline__ half8_t q4k_bop(const WTile& w, const WScale& c, int 
 // DIRECT (an unsplit plan of one tensor): the rows below tg.row_end go to the
 // caller's output.  An instantiation of its own: a test at every store of
 // the partials makes each a branch, for rows that the engine always pads.
+// With one activation tile and one weight tile a wave, every fourth block's
+// sum moves to a second accumulator, so that a row's sums are those of splits of
+// DEC_BPS_OP blocks (with two weight tiles its registers leave a wave less a
+// SIMD: 128256 x 4096, 16 rows, row layout 78 -> 89 us; call_plan sees to it).
 template <int R, bool TILED, int WAVES = 4, int NT = 1, bool CONV = false, bool DIRECT = false>
 __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, const uint4* frag,
                                                              float* __restrict__ out, int64_t ldo,
@@ -235,6 +243,7 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, cons
                                                              const float* X = nullptr, int64_t ldx = 0,
                                                              int xrows = 0) {
     static_assert(!CONV || (NT == 1 && WAVES == 8), "CONV: one activation tile, two rows per wave");
+    constexpr bool FOLD = DIRECT && NT == 1 && R == 1;
     __shared__ uint4 s_act[2 * NT * ACT_FRAG_UNITS];
     constexpr int TCH = ACT_FRAG_UNITS / 64;          // 1 KiB wave copies per tile and block
     constexpr int CHUNKS = NT * TCH;
@@ -282,11 +291,13 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, cons
         }
     };
     WTile w0[R], w1[R];
-    floatx4 acc[R][NT];
+    floatx4 acc[R][NT], tot[FOLD ? R : 1];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+    for (int r = 0; r < R; ++r) {
+        if constexpr (FOLD) tot[r] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[r][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
 
     // a block's products from the landed weights wc and operand buffer slot
     auto compute = [&](const WTile (&wc)[R], int slot) {
@@ -350,6 +361,13 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, cons
     auto step = [&](const WTile (&wc)[R], WTile (&wn)[R], int b) {
         if (b + 1 < nb) issue(wn, b + 1);            // the last block prefetches nothing
         compute(wc, b & 1);
+        if constexpr (FOLD)
+            if (b % DEC_BPS_OP == DEC_BPS_OP - 1)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    tot[r] += acc[r][0];
+                    acc[r][0] = floatx4{0.f, 0.f, 0.f, 0.f};
+                }
         __builtin_amdgcn_sched_barrier(0);
         SH_WAIT_VMCNT(0);                              // block b+1's units and weights have landed
         __syncthreads();
@@ -437,6 +455,7 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_dec_kernel(Q4kTargets tg, cons
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int row = (tile0 + r) * 16 + j;
+        if constexpr (FOLD) acc[r][0] = tot[r] + acc[r][0];
         if (tile0 + r < tiles && row < M) {
 #pragma unroll
             for (int n = 0; n < NT; ++n)
@@ -806,15 +825,14 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_pf_kernel(Q4kTargets tg, const
 // R 1 / S 4, O R 1 / S 8, gate+up R 2 / S 2, down R 1 / S 8 and the LM head
 // R 2 / S 1, each the fastest decode step of the per-shape choices measured
 // (decode step -1.5 to -1.8 % against a largest-R-first rule at the same
-// target).  The C ABI's matmul of 2-16 rows, whose partials only a split
-// sum reads, allows 4 (14336x4096 at 16 rows: 16.9 vs 21.3 us with 8).
+// target).  The C ABI's matmul of 2-16 rows that converts its activations,
+// whose partials only a split sum reads, allows 4 (14336x4096 at 16 rows:
+// 16.9 vs 21.3 us with 8); on an operand see call_plan.
 // Splits keep >= 2 blocks each: a one-block split never overlaps its weight
 // prefetch with compute.  Waves per decode workgroup: 8 by default
 // (measured 2 % faster per decode step than 4, since each staged activation
 // block feeds twice the weight tiles, and 16 was 8 % slower);
 // SLATE_HIP_Q4K_W=4 selects four.
-constexpr int DEC_BPS_STEP = 8, DEC_BPS_OP = 4;
-
 static int dec_waves() {
     return knobs().q4k_w;
 }
@@ -850,6 +868,30 @@ static void dec_plan(const int* tiles, int n, int nblk, int s_max, int bps_max, 
     if (S_env > 0) S_out_v = S_env < s_max ? S_env : s_max;
     *R_out = R_out_v;
     *S_out = S_out_v;
+}
+
+// The C ABI's plan of 2-16 rows on an operand: the engine's, unless a row's sum
+// would pass through more additions than with splits of DEC_BPS_OP blocks (a
+// split's blocks one after the other, then the splits; unsplit, the kernel
+// adds every DEC_BPS_OP blocks apart).  14336 x 4096: splits of 8 blocks show
+// 3.986e-7 against 64 bits, of 4 3.979e-7, the same bits as the converting
+// kernel's; 16 rows 17.0 and 16.3 us, 20.9 and 19.1 on weights the caches have
+// not seen.  10240 x 8192 keeps splits of 8 (12 additions either way; 24.3 and
+// 25.0 us, tiled 19.3 and 21.9).
+static void call_plan(int tiles, int nblk, int s_max, int* R, int* S) {
+    dec_plan(&tiles, 1, nblk, s_max, DEC_BPS_STEP, R, S);
+    if ((nblk + *S - 1) / *S <= DEC_BPS_OP) return;   // the other plan is the same
+    int Ro, So;
+    dec_plan(&tiles, 1, nblk, s_max, DEC_BPS_OP, &Ro, &So);
+    if (So == 1) return;                              // unsplit either way
+    auto sums = [&](int r, int s) {
+        const int bps = s == 1 && r == 1 ? DEC_BPS_OP : (nblk + s - 1) / s;
+        return bps + (nblk + bps - 1) / bps;
+    };
+    if (sums(*R, *S) > sums(Ro, So)) {
+        *R = Ro;
+        *S = So;
+    }
 }
 
 template <int R, bool TILED, int NT, bool DIRECT>
@@ -1013,7 +1055,8 @@ int launch_q4k(const Q4kTarget* t, int n, bool tiled, const Act16& a, float* out
     int tiles[3];
     for (int i = 0; i < n; ++i) tiles[i] = (t[i].M + 15) / 16;
     int R, S;
-    dec_plan(tiles, n, nblk, max_splits, DEC_BPS_STEP, &R, &S);
+    if (direct && act_tiles == 1) call_plan(tiles[0], nblk, max_splits, &R, &S);
+    else dec_plan(tiles, n, nblk, max_splits, DEC_BPS_STEP, &R, &S);
     const int bps = (nblk + S - 1) / S;
     S = (nblk + bps - 1) / bps;                       // every split gets >= 1 block
     Q4kTargets tg{};
@@ -1058,12 +1101,17 @@ static void launch_dec_conv(const Q4kTargets& tg, const float* X, int64_t ldx, i
 // itself.  The operand pays where the plan on it is unsplit (then it writes
 // the final rows: two launches either way; 128256 x 4096 at 16 rows 97 -> 69
 // us, 32000 x 2048 15.9 -> 12.7), and where the matmul is long enough: from
-// 28672 x 4096 at any row count (2 rows 24.7 -> 19.7 us), at 13-16 rows from
-// 14336 x 4096 (15.9 -> 14.5 us; 4096 x 11008 15.1 -> 15.9, so not there).
+// 28672 x 4096 at any row count (2 rows 24.7 -> 19.7 us), and at 13-16 rows from
+// 14336 x 4096 where at least 40 column groups of 128 repeat the conversion
+// (tiled, 16 rows, on weights the caches have not seen: 14336 x 4096 16.8 ->
+// 16.2 us, 8192 x 8192 18.2 -> 18.3, 13824 x 5120 19.9 -> 18.4; 4096 x 14336, 32
+// groups, 18.9 -> 19.5 and on the row layout 20.9 -> 22.6; 4096 x 11008 15.1 ->
+// 15.9).
 bool q4k_conv_pays(int rows, int M, int K) {
-    int tiles = (M + 15) / 16, R, S;
-    dec_plan(&tiles, 1, K / QK, 32, DEC_BPS_STEP, &R, &S);
-    return S > 1 && (double)M * K < (rows > 12 ? 50.0 : 80.0) * 1048576.0;
+    const double mk = (double)M * K / 1048576.0;
+    int R, S;
+    call_plan((M + 15) / 16, K / QK, 32, &R, &S);
+    return S > 1 && mk < 80.0 && !(rows > 12 && mk >= 50.0 && M >= 40 * 128);
 }
 
 int launch_q4k_conv(const Q4kTarget& t, bool tiled, const float* X, int64_t ldx, int rows, int K, float* out,

@@ -198,6 +198,26 @@ def test_q4k_rows_of_the_output(hip, B, M, K, form):
     assert np.all(np.abs(got[:B * M].reshape(B, M) - X6 @ w.T) <= bound)
 
 
+# 13-16 rows of a long matmul go over an operand, fewer through the converting
+# kernel: at these shapes both add up the same values in the same splits, so
+# a row's result has the same bits either way.
+@pytest.mark.parametrize("M,K", [(14336, 4096), (18944, 3584), (13000, 4352)])
+def test_q4k_rows_the_same_over_operand_and_conversion(hip, M, K):
+    rng = np.random.default_rng(M + K)
+    raw, _, _ = _q4k(rng, M, K)
+    X = rng.normal(0, 1, (16, K)).astype(np.float32)
+    A, Xd, Y = DB.from_array(raw), DB.from_array(X), DB(16 * M * 4)
+    T = DB(hip.lib.slate_hip_q4k_tiled_bytes(M, K))
+    check(hip.lib.slate_hip_q4k_tile(T.p, A.p, M, K), "q4k_tile")
+    for fn, w in ((hip.lib.slate_hip_matmul_q4k, A), (hip.lib.slate_hip_matmul_q4k_tiled, T)):
+        got = {}
+        for B in (7, 12, 13, 16):
+            check(fn(Y.p, w.p, Xd.p, B, M, K), "matmul_q4k")
+            got[B] = host(Y, (16, M))[:B].view(np.uint32).copy()
+        for B in (7, 12, 13):
+            assert np.array_equal(got[B], got[16][:B]), B
+
+
 # One row: x handed out through LDS (from 6M weights on) and loaded directly,
 # with whole and partly filled waves of blocks, one and two passes over K, and
 # the 16-row workgroups of long rows.
