@@ -378,8 +378,10 @@ static int matmul_q8_common(float* Y, const void* A, const float* X, int B, int 
     SH_REQUIRE(Y && A && X && B > 0 && M > 0 && K > 0, "matmul_q8_0: bad arguments");
     SH_REQUIRE(K % Q8_ELEMS == 0, "matmul_q8_0: K=%d is not a multiple of 32", K);
     std::lock_guard<std::mutex> lk(g_enqueue_mu);
-    // one row: one kernel straight into Y (no operand, no partials)
-    if (B == 1) return launch_q8_gemv(A, tiled, M, K, X, Y, g_stream);
+    // one row: one kernel straight into Y (no operand, no partials), unless
+    // it would write the row that its other workgroups still read
+    const bool apart = Y + M <= X || X + K <= Y;
+    if (B == 1 && apart) return launch_q8_gemv(A, tiled, M, K, X, Y, g_stream);
     const void* W = A;
     int rc;
     if (!tiled) {   // regroup the row layout into the matmul's tiles first

@@ -108,6 +108,28 @@ def test_q8_row_layout_edges(hip, B, M, K):
     assert np.all(np.abs(got - X6 @ w.T) <= bound)
 
 
+# One row into its own memory (whole, or its second half): every result is
+# made from the row as it came, as where the results go elsewhere.
+@pytest.mark.parametrize("M,K,off", [(4096, 4096, 0), (14336, 4096, 2048), (2048, 8192, 4096)])
+def test_q8_matvec_over_its_own_row(hip, M, K, off):
+    rng = np.random.default_rng(M + K)
+    raw, w = _q8(rng, M, K)
+    x = rng.normal(0, 1, K).astype(np.float32)
+    A, T = DB.from_array(raw), DB(hip.lib.slate_hip_q8_0_tiled_bytes(M, K))
+    check(hip.lib.slate_hip_q8_0_tile(T.p, A.p, M, K), "q8_0_tile")
+    x6 = x.astype(np.float64)
+    # (the bound of test_q8_row_layout_edges for more than one row)
+    xmax = np.repeat(np.abs(x6).reshape(-1, 256).max(-1), 256)
+    bound = (K // 32 * 18 + 32) * EPS * (np.abs(w) @ np.abs(x6)) + 2.0 ** -22 * (np.abs(w) @ xmax)
+    for fn, weights in ((hip.lib.slate_hip_matmul_q8_0, A), (hip.lib.slate_hip_matmul_q8_0_tiled, T)):
+        for _ in range(3):
+            buf = DB((K + M) * 4)
+            buf.upload(x)
+            check(fn(buf.ptr + 4 * off, weights.p, buf.p, 1, M, K), "matmul_q8_0")
+            got = host(buf, (K + M,))[off:off + M]
+            assert np.all(np.abs(got - w @ x6) <= bound)
+
+
 # Widths around the one-, two- and four-float4 forms (4096, 8192, 16384), odd
 # widths and rows that start off 16 bytes (the plain form); y may be x.
 @pytest.mark.parametrize("D,off", [(1, 0), (3, 0), (4, 0), (256, 1), (260, 0), (4096, 0), (4100, 0), (8192, 0),
