@@ -188,7 +188,8 @@ int   slate_hip_pack_batch(const int32_t* slot, const int32_t* pos0, const int32
  * q      : [T, n_q_heads*hd] post-RoPE queries, packed token-major
  * kv     : K and V pools; the cache of kv head h of the sequence that owns
  *          token t starts at kv_base[tok2seq[t]] + h*head_stride and holds
- *          [max_seq, hd] rows (key position-major)
+ *          [max_seq, hd] rows (key position-major); any float offset is
+ *          taken, rows that start on 16 bytes are read fastest
  * token t attends to key positions 0..tok_pos[t] of its own sequence.
  * out    : [T, n_q_heads*hd].  scale = 1/sqrtf(hd) as llama_infer.c:104. */
 int   slate_hip_attention_ragged(float* out, const float* q, const float* Kpool,

@@ -1,7 +1,8 @@
 // k_q4k_gemv.hip -- Q4_K matrix-vector products for 1..4 activation rows on
 // the vector ALUs: slate_q4_k_matvec (src/util/quant.c:306-313) for a small
-// batch, with no activation operand conversion, no LDS staging of
-// activations and no split-K partials (one kernel writes the final rows).
+// batch, with no activation operand conversion and no split-K partials (one
+// kernel writes the final rows).  One activation row passes through LDS from
+// about 6M weights on (XLDS below); otherwise the threads load theirs.
 //
 // Work split.  A workgroup owns R weight rows and all of K.  Thread t owns
 // sub-block s = t & 7 of super-block kb = t >> 3 (32 elements of K): its

@@ -403,10 +403,12 @@ __global__ __launch_bounds__(64 * WAVES) void q8_mm_kernel(Q4kTargets tg, const 
 // DPP over the wave and LDS over the waves in wave order: deterministic, and
 // the same bits from both layouts.
 //
-// Bound by HBM and by the latency of the one round of loads.  Per call at
-// 4096 x 4096, row layout: 46.9 us as regrouping pass + operand + matmul +
-// split sum, 5.7 us as one kernel; TILED 11.6 us as operand + matmul + split
-// sum, 6.9 us; 14336 x 4096: 129 and 17.7 us, 12.3 (5.1 TB/s) and 16.5 us.
+// Bound by the latency of the one round of loads and by reading W.  Per call at
+// 4096 x 4096, row layout: 47.2 us as regrouping pass + operand + matmul +
+// split sum, 5.7-6.1 us as one kernel; TILED 11.6 us as operand + matmul +
+// split sum, 5.5 us; 14336 x 4096: 129 and 18.0 us, 12.8 and 14.2 us.  These
+// repeat one W, which the Infinity Cache holds; on copies that it does not,
+// 47.7 -> 7.6, 12.8 -> 8.1, 130 -> 18.4 (3.4 TB/s) and 20.4 -> 19.3 us.
 constexpr int Q8V_WAVES = 8;
 template <int R, bool TILED>
 __global__ __launch_bounds__(64 * Q8V_WAVES) void q8_gemv_kernel(const uint8_t* __restrict__ W,

@@ -839,10 +839,12 @@ int launch_mm_f32(float* Y, const float* X, const float* W, int B, int M, int K,
 // shuffle.  The waves' sums meet in LDS and are added in wave order.
 //
 // What bounds it: reading W once from 8192 columns on (4096 x 16384 at B 16:
-// 53 us, 5.1 TB/s), below that latency and the MFMAs of the few CUs that have
+// 53 us, 5.1 TB/s over copies of W that the caches have not seen, 42 us on the
+// same W again), below that latency and the MFMAs of the few CUs that have
 // a workgroup.  The form before (a column per lane, four waves over k, one
 // dependent load of W and one of X per batch row and k) took 208 us per call
-// for B 16, K 1024, N 4096, this one 6.8 us.
+// for B 16, K 1024, N 4096, this one 6.8 us (on copies that the caches have not
+// seen 232 and 9.5).
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // rows start on any float
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef float fx4 __attribute__((ext_vector_type(4)));
@@ -967,7 +969,8 @@ static void launch_linear(float* C, const float* X, const float* W, int B, int K
 // two, then four (wider runs of W, fewer reads of X): K 1024, N 4096, B 16
 // takes 6.8 us with one, 8.8 with two, 11.2 with four; K 2048, N 8192 16.7 /
 // 15.3 / 19.7; K 4096, N 16384 94 / 62 / 53 us.  Waves and units in flight
-// keep two workgroups' registers on a CU.
+// keep two workgroups' registers on a CU; with four columns and more than 32
+// rows the waves' sums take 128 of its 160 KiB of LDS, and one workgroup fits.
 template <int BT, int NW>
 static void launch_linear_cols(float* C, const float* X, const float* W, int B, int K, int N, hipStream_t s) {
     constexpr int A = BT == 1 ? 4 : 2;

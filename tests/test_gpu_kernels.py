@@ -480,7 +480,8 @@ def test_attention_ragged_vs_oracle(hip, orc, hd, Hq, Hkv, extra):
     """Per-token GQA attention over ragged per-sequence caches, one query per
     token (decode) and several consecutive queries of one sequence (prefill
     chunk), lengths across chunk boundaries.  `extra` adds a 70-token prompt
-    chunk (launches of more than 64 query tokens take the phased kernel)."""
+    chunk (calls of more than 64 query tokens whose tokens share keys take the
+    run kernel)."""
     lib = load_library()
     rng = np.random.default_rng(hd + Hq)
     max_seq = 4352
